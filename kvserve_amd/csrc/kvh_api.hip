@@ -71,10 +71,11 @@ Plan make_plan(int64_t T, int32_t B, int32_t H, int32_t Hkv, int32_t D, int32_t 
     const size_t prows = pl.launch_prefill ? (size_t)2 * kMaxPrefillUnits * kPrefillRows : 0;
     pl.ws_pacc_bytes = align_up(prows * D * sizeof(float));
     pl.ws_pml_bytes = align_up(prows * 2 * sizeof(float));
-    // plan: header, sequence list, flat starts, unit starts
+    // where each prefill unit starts, behind a header and two per-sequence arrays that no kernel
+    // uses any more: callers size their workspaces by this sum, which stays
     pl.ws_plan_bytes = pl.launch_prefill ? align_up(4 * sizeof(int64_t)) + align_up((size_t)B * sizeof(int32_t)) +
                                                align_up(((size_t)B + 1) * sizeof(int64_t)) +
-                                               align_up((size_t)kMaxPrefillUnits * kPreRec * sizeof(int32_t))
+                                               align_up((size_t)kMaxPrefillUnits * kPreStartBytes)
                                          : 0;
     // cascade over a shared prefix: share header, decode list, prefix partials, merge jobs
     pl.cascade = !pl.launch_prefill && pl.NT == 1 && B >= 2 && (int64_t)W * BS > kCascadeMinTokens;
@@ -433,16 +434,8 @@ static int paged_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_h
     w += plan.ws_pacc_bytes;
     p.ws_pml = plan.ws_pml_bytes ? (float*)w : nullptr;
     w += plan.ws_pml_bytes;
-    if (plan.ws_plan_bytes) {
-      p.ws_plan_hdr = (int64_t*)w;
-      w += align_up(4 * sizeof(int64_t));
-      p.ws_pre_list = (int32_t*)w;
-      w += align_up((size_t)num_seqs * sizeof(int32_t));
-      p.ws_pre_beg = (int64_t*)w;
-      w += align_up(((size_t)num_seqs + 1) * sizeof(int64_t));
-      p.ws_pre_unit = (int32_t*)w;
-      w += align_up((size_t)kMaxPrefillUnits * kPreRec * sizeof(int32_t));
-    }
+    p.ws_plan = plan.ws_plan_bytes ? w : nullptr;
+    w += plan.ws_plan_bytes;
     if (plan.ws_x_bytes) {
       const size_t rows = (size_t)plan.xrows;
       p.ws_share = (int64_t*)w;

@@ -33,10 +33,12 @@
 //    direct global->LDS loads, each wave computing 32 query rows.
 // Grids depend only on static shapes and the device's occupancy, never on per-step
 // lengths, so every launch is HIP-graph capturable.
+#include <algorithm>
 #include <type_traits>
 
 #include "kvh_device.h"
 #include "kvh_internal.h"
+#include "prefill_plan.h"
 
 namespace kvh {
 
@@ -833,9 +835,7 @@ constexpr int64_t kPrefix64Cost = 11, kChunkCost = 8;
 // grid 2-7% slower with 4/3 and keep equal shares.
 constexpr int64_t kRound1Share = 4, kRound2Share = 3;
 
-constexpr int kPlanThreads = 256;    // the decode kernel's workgroup
-constexpr int kPlanLdsSeqs = 1024;  // flat starts kept in LDS for the unit search (else global)
-__device__ void plan_prefill(const PAParams& p);
+constexpr int kPlanThreads = 256;  // a workgroup of the kernels that scan the batch
 
 // ---------------------------------------------------------------------------------------
 // Cascade decode over a shared prefix (prefix caching hands several sequences the same
@@ -1020,19 +1020,14 @@ __device__ __forceinline__ void write_job_x(int32_t* job, int pieces, int64_t sl
   job[0] = kJobDecode;
 }
 
-// Decode class: grid (NU * HGW / 4) workgroups of 4 waves; wave w of workgroup b is head
-// w % HGW of unit (4 b + w) / HGW. In mixed batches (PLAN) workgroup 0 computes the prefill
-// plan instead and the units start at workgroup 1. KV8: the cache is E4M3. NX: 16-row tiles
-// of a cascade prefix group (XR = 16 NX rows; 1 outside the cascade).
+// Decode class: NU * HGW / 4 workgroups of 4 waves; wave w of workgroup `block` is head w % HGW
+// of unit (4 block + w) / HGW. KV8: the cache is E4M3. NX: 16-row tiles of a cascade prefix
+// group (XR = 16 NX rows; 1 outside the cascade).
 template <class E, int D, int NT, bool KV8, int NX>
-__global__ __launch_bounds__(256) void pa_decode_kernel(PAParams p) {
-  if (p.PLAN && blockIdx.x == 0) {
-    plan_prefill(p);
-    return;
-  }
+__device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int gw = (blockIdx.x - (p.PLAN ? 1 : 0)) * kWavesPerWG + wave;
+  const int gw = block * kWavesPerWG + wave;
   const int unit = gw / p.HGW;
   // With two workgroups per CU, the second-round units (unit >= R1, each sharing its CUs with
   // a first-round unit) take the two head halves the other way round, so every CU reads both
@@ -2108,128 +2103,153 @@ __device__ __forceinline__ void prefill_tile_kv8(char* lds, const PAParams& p, c
   pf_write_rows<E, D, NT>(s, p, sv, R, row0, kvh, partial, slot * PRW - wg_row0);
 }
 
-// Chunks of tile t (rows 128 t .. of R): those its last row can see, at least one so that
-// every tile is visited and written.
-__device__ __forceinline__ int pre_tile_chunks(const PAParams& p, const SeqView& sv, int R, int t) {
-  const int last = min(p.PR * t + p.PR - 1, R - 1);
-  const int lim = (int)clamp64(sv.ctx + last / p.G + 1, 0, sv.kv_total);
-  return max(1, (lim + kChunk - 1) / kChunk);
+__device__ __forceinline__ PreSeq pre_seq(const PAParams& p, const SeqView& sv) {
+  return PreSeq{sv.q_len * p.G, sv.q_len, sv.kv_total, sv.ctx};
 }
 
-// Fixed cost of a tile (Q load, pipeline fill, output write) in chunk steps: each tile
-// occupies kTileCost + chunks positions of the flat space, the first kTileCost virtual.
-constexpr int kTileCost = 4;
+__device__ __forceinline__ int pre_tile_chunks(const PAParams& p, const SeqView& sv, int R, int t) {
+  return pre_tile_chunks(PreSeq{R, sv.q_len, sv.kv_total, sv.ctx}, p.G, p.PR, t);
+}
 
 // Flat positions of all tiles of one kv head of a prefill-class sequence; 0 for others.
-__device__ __forceinline__ int64_t pre_seq_chunks(const PAParams& p, const SeqView& sv) {
+template <int PR>
+__device__ __forceinline__ int64_t pre_seq_positions(const PAParams& p, const SeqView& sv, int step) {
   if (sv.q_len <= p.QS) return 0;
-  const int R = sv.q_len * p.G;
-  const int tiles = (R + p.PR - 1) / p.PR;
-  int64_t n = 0;
-  for (int t = 0; t < tiles; ++t) n += kTileCost + pre_tile_chunks(p, sv, R, t);
-  return n;
+  const PreSeq s = pre_seq(p, sv);
+  return pre_prefix(s, p.G, PR, step, (s.R + PR - 1) / PR);
 }
 
-// Prefill plan, computed by workgroup 0 of the decode launch in mixed batches (so it runs
-// under the decode work instead of ahead of it): the list of prefill-class sequences, the
-// flat start of each (prefix sums of Hkv x pre_seq_chunks) and, for each prefill workgroup,
-// a record of where its unit starts (below). Every prefill workgroup then starts from one
-// scalar load of its record instead of scanning the batch or chasing the unit -> sequence
-// -> lengths chain through memory.
-__device__ void plan_prefill(const PAParams& p) {
-  __shared__ int64_t s_pos[kPlanThreads];
-  __shared__ int32_t s_cnt[kPlanThreads];
-  __shared__ int64_t s_beg[kPlanLdsSeqs + 1];
-  const int tid = threadIdx.x;
+// x / y of non-negative wave-uniform values, in 32 bits where they fit.
+__device__ __forceinline__ int64_t div_uniform(int64_t x, int64_t y) {
+  return ((uint64_t)x | (uint64_t)y) >> 32 ? x / y : (int64_t)((uint32_t)x / (uint32_t)y);
+}
+
+__device__ __forceinline__ int64_t readlane64(int64_t x, int l) {
+  return ((int64_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+}
+
+// The first prefill-class sequence at or after `from` (B when there is none), 64 at a time.
+__device__ __forceinline__ int next_prefill_seq(const PAParams& p, int from) {
+  const int lane = threadIdx.x & 63;
+  for (int s0 = from; s0 < p.B; s0 += 64) {
+    const int sq = s0 + lane;
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(sq < p.B && seq_view(p, min(sq, p.B - 1)).q_len > p.QS);
+    if (hit) return s0 + __builtin_ctzll(hit);
+  }
+  return p.B;
+}
+
+// Where a prefill workgroup's unit starts, computed by the workgroup itself (LDS: PreStart
+// and one word per wave): its 256 threads each add up the flat positions of B / 256 sequences, a
+// block scan gives the size C of the flat space, and the wave whose range holds the unit's
+// first position finds the sequence, kv head and tile there, trying 64 tiles at a time.
+struct alignas(16) PreStart {
+  int64_t C, x0, x1, qs, ctx;
+  int32_t u, t, rem, q_len, kv_total;
+  uint16_t seq, kvh;  // at most 65535 of each (checked on the host)
+};
+static_assert(sizeof(PreStart) == kPreStartBytes, "the workspace holds one per prefill unit");
+
+template <int PR>
+__device__ __forceinline__ bool prefill_start(const PAParams& p, int b, PreStart* st, int64_t* wsum) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int per = (p.B + kPlanThreads - 1) / kPlanThreads;
   const int s0 = min(tid * per, p.B), s1 = min(s0 + per, p.B);
+  const int step = PR % p.G == 0 ? PR / p.G : 0;
+  SeqView sv{};  // this thread's last sequence: the only one in batches of up to 256
   int64_t pos = 0;
-  int cnt = 0;
   for (int sq = s0; sq < s1; ++sq) {
-    const int64_t c = (int64_t)p.Hkv * pre_seq_chunks(p, seq_view(p, sq));
-    pos += c;
-    cnt += c > 0;
+    sv = seq_view(p, sq);
+    pos += (int64_t)p.Hkv * pre_seq_positions<PR>(p, sv, step);
   }
-  s_pos[tid] = pos;
-  s_cnt[tid] = cnt;
+  int64_t incl = pos;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int64_t y = __shfl_up(incl, o);
+    if (lane >= o) incl += y;
+  }
+  if (lane == 63) wsum[wv] = incl;
   __syncthreads();
-  for (int o = 1; o < kPlanThreads; o <<= 1) {  // inclusive scan over the threads' ranges
-    const int64_t a = tid >= o ? s_pos[tid - o] : 0;
-    const int b = tid >= o ? s_cnt[tid - o] : 0;
-    __syncthreads();
-    s_pos[tid] += a;
-    s_cnt[tid] += b;
-    __syncthreads();
+  int64_t beg = incl - pos, C = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) {
+    const int64_t x = wsum[w];
+    if (w < wv) beg += x;
+    C += x;
   }
-  const int64_t C = s_pos[kPlanThreads - 1];
-  const int n_pre = s_cnt[kPlanThreads - 1];
-  int64_t beg = s_pos[tid] - pos;
-  int k = s_cnt[tid] - cnt;
-  for (int sq = s0; sq < s1; ++sq) {
-    const int64_t c = (int64_t)p.Hkv * pre_seq_chunks(p, seq_view(p, sq));
-    if (c > 0) {
-      p.ws_pre_list[k] = sq;
-      p.ws_pre_beg[k] = beg;
-      if (k < kPlanLdsSeqs) s_beg[k] = beg;
-      beg += c;
-      ++k;
+  C = uni64(C);
+  if (C == 0) return false;
+  const int NUa = (int)active_units(C, p.NUP);
+  // workgroup b's unit, XCD by XCD (b % 8), then b / 8
+  const int q8 = NUa / 8, r8 = NUa % 8, xcd = b % 8, jj = b / 8;
+  if (jj >= q8 + (xcd < r8 ? 1 : 0)) return false;  // idle workgroup (workgroup-uniform)
+  const int u = xcd * q8 + min(xcd, r8) + jj;
+  const int64_t x0 = div_uniform((int64_t)u * C, NUa);
+  const uint64_t own = __builtin_amdgcn_ballot_w64(beg <= x0 && x0 < beg + pos);  // one thread of one wave
+  if (own) {  // that wave, in scalar code (wave-uniform)
+    const int l = __builtin_ctzll(own);
+    int sq = __builtin_amdgcn_readlane(s0, l);
+    int64_t off = x0 - readlane64(beg, l), per_kvh;
+    SeqView v;
+    if (per == 1) {
+      v.qs = readlane64(sv.qs, l);
+      v.ctx = readlane64(sv.ctx, l);
+      v.q_len = __builtin_amdgcn_readlane(sv.q_len, l);
+      v.kv_total = __builtin_amdgcn_readlane(sv.kv_total, l);
+      per_kvh = div_uniform(readlane64(pos, l), p.Hkv);
+    } else {
+      const int end = __builtin_amdgcn_readlane(s1, l);
+      for (;; ++sq) {
+        v = seq_view_uniform(p, sq);
+        per_kvh = uni64(pre_seq_positions<PR>(p, v, step));
+        if (off < p.Hkv * per_kvh || sq + 1 >= end) break;
+        off -= p.Hkv * per_kvh;
+      }
     }
-  }
-  const int NUa = C > 0 ? (int)active_units(C, p.NUP) : 0;
-  if (tid == 0) {
-    p.ws_plan_hdr[0] = C;
-    p.ws_plan_hdr[1] = NUa;
-    p.ws_plan_hdr[2] = n_pre;
-    p.ws_pre_beg[n_pre] = C;
-    if (n_pre <= kPlanLdsSeqs) s_beg[n_pre] = C;
-  }
-  __syncthreads();  // the list and starts are visible to the whole workgroup
-  const int64_t* beg_tab = n_pre <= kPlanLdsSeqs ? s_beg : p.ws_pre_beg;
-  const int q8 = NUa / 8, r8 = NUa % 8;
-  for (int b = tid; b < p.NUP; b += kPlanThreads) {
-    // workgroup b's unit, as prefill_units deals them: XCD by XCD (b % 8), then b / 8
-    const int xcd = b % 8, jj = b / 8;
-    int32_t* d = p.ws_pre_unit + (int64_t)b * kPreRec;
-    if (NUa == 0 || jj >= q8 + (xcd < r8 ? 1 : 0)) {
-      d[0] = -1;  // idle, rewritten on every call
-      continue;
-    }
-    const int u = xcd * q8 + min(xcd, r8) + jj;
-    const int64_t x0 = u * C / NUa;
-    int lo = 0, hi = n_pre - 1;  // last sequence starting at or before x0
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) / 2;
-      if (beg_tab[mid] <= x0)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const int seq = p.ws_pre_list[lo];
-    const SeqView sv = seq_view(p, seq);
-    const int R = sv.q_len * p.G;
-    const int64_t per_kvh = (beg_tab[lo + 1] - beg_tab[lo]) / p.Hkv;
-    const int64_t off = x0 - beg_tab[lo];
-    const int kvh = (int)(off / per_kvh);
-    int64_t rem = off % per_kvh;
+    const int kvh = (int)div_uniform(off, per_kvh);
+    off -= kvh * per_kvh;
+    // the tile: the last one that starts at or before off
+    const PreSeq s = pre_seq(p, v);
+    const int tiles = (s.R + PR - 1) / PR;
     int t = 0;
-    for (int n_t = pre_tile_chunks(p, sv, R, 0); rem >= kTileCost + n_t; n_t = pre_tile_chunks(p, sv, R, t)) {
-      rem -= kTileCost + n_t;
-      ++t;
+    int64_t t_beg = 0;
+    for (int t0 = 0; t0 < tiles; t0 += 64) {
+      const int64_t x = pre_prefix(s, p.G, PR, step, min(t0 + lane, tiles));
+      const uint64_t le = __builtin_amdgcn_ballot_w64(t0 + lane < tiles && x <= off);
+      if (le == 0) break;
+      const int k = 63 - __builtin_clzll(le);
+      t = t0 + k;
+      t_beg = readlane64(x, k);
+      if (k < 63) break;
     }
-    const int64_t x1 = (u + 1) * C / NUa;
-    d[1] = lo;
-    d[2] = kvh;
-    d[3] = t;
-    d[4] = (int)rem;  // < kTileCost + chunks of one tile
-    d[5] = seq;
-    d[6] = sv.q_len;
-    d[7] = sv.kv_total;
-    *(int64_t*)(d + 8) = sv.qs;
-    *(int64_t*)(d + 10) = sv.ctx;
-    *(int64_t*)(d + 12) = x0;
-    *(int64_t*)(d + 14) = x1;
-    d[0] = u;
+    if (lane == 0)
+      *st = PreStart{C, x0, div_uniform((int64_t)(u + 1) * C, NUa), v.qs, v.ctx, u, t, (int)(off - t_beg), v.q_len,
+                     v.kv_total, (uint16_t)sq, (uint16_t)kvh};
   }
+  __syncthreads();
+  return true;
+}
+
+// In a mixed batch's own decode launch NUP more workgroups follow the decode units (grid (NU HGW
+// / 4) + NUP): each writes where a prefill unit starts, under the decode work, and the prefill
+// launch behind it begins with one load. (Computed by the prefill workgroups themselves it was
+// on that launch's path: 512 decodes and four 384-token chunks over E4M3 caches 483 -> 492 us.)
+template <class E, int D, int NT, bool KV8, int NX>
+__global__ __launch_bounds__(256) void pa_decode_kernel(PAParams p) {
+  const int b = blockIdx.x;
+  if constexpr (NX == 1) {
+    if (p.ND > 0 && b >= p.ND) {
+      __shared__ PreStart st;
+      __shared__ int64_t wsum[kPlanThreads / 64];
+      const bool work = prefill_start<kWavesPerWG * 16 * prefill_nt<KV8>()>(p, b - p.ND, &st, wsum);
+      if (threadIdx.x == 0) {
+        if (!work) st.u = -1;  // idle, rewritten on every call
+        ((PreStart*)p.ws_plan)[b - p.ND] = st;
+      }
+      return;
+    }
+  }
+  decode_unit<E, D, NT, KV8, NX>(p, b);
 }
 
 // Stream-K over the prefill-class work: a flat space of (sequence, kv head, tile, chunk),
@@ -2244,35 +2264,34 @@ __device__ void plan_prefill(const PAParams& p) {
 // dealt to the 8 XCDs round-robin, so the units are numbered XCD by XCD: the units of one
 // XCD are contiguous in the flat space and read the same sequence's K/V through that
 // XCD's L2.
-// The units' walk over the flat space (shared by both prefill kernels): `tile(sv, R, seq,
-// kvh, t, c_lo, c_hi, partial, slot, rest, total)` computes chunks [c_lo, c_hi) of tile t.
-template <class TileFn>
-__device__ __forceinline__ void prefill_units(const PAParams& p, TileFn&& tile) {
-  // this workgroup's record (one 64-byte load) and the plan header, issued together and
-  // ahead of any store
-  static_assert(kPreRec == 16, "one i32x16 per record");
-  const i32x16 rec = *(const i32x16*)(p.ws_pre_unit + (int64_t)blockIdx.x * kPreRec);
-  const int64_t hdr_c = p.ws_plan_hdr[0], hdr_nua = p.ws_plan_hdr[1], hdr_npre = p.ws_plan_hdr[2];
-  int32_t* job = p.ws_job + (int64_t)(kMaxDecodeWaves + blockIdx.x) * kJobInts;
+// The walk of workgroup b's unit over the flat space (shared by both prefill tiles): `tile(sv,
+// R, seq, kvh, t, c_lo, c_hi, partial, slot, rest, total)` computes chunks [c_lo, c_hi) of tile t.
+// PLANNED: the start is in the workspace (pa_decode_kernel); else it is computed here, in lds,
+// which is free again when the first tile is computed.
+template <int PR, bool PLANNED, class TileFn>
+__device__ __forceinline__ void prefill_units(const PAParams& p, int b, char* lds, TileFn&& tile) {
+  int32_t* job = p.ws_job + (int64_t)(kMaxDecodeWaves + b) * kJobInts;
   if (threadIdx.x == 0) job[0] = kJobNone;
-  const int u = uni(rec[0]);
-  if (u < 0) return;  // idle workgroup (workgroup-uniform)
-  const int64_t C = uni64(hdr_c);
-  const int NUa = (int)uni64(hdr_nua);
-  const int n_pre = (int)uni64(hdr_npre);
-  const auto pair = [&](int i) { return (int64_t)(((uint64_t)(uint32_t)rec[i + 1] << 32) | (uint32_t)rec[i]); };
-  int k = uni(rec[1]);
-  int kvh = uni(rec[2]);
-  int t = uni(rec[3]);
-  int64_t rem = uni(rec[4]);
-  int seq = uni(rec[5]);
+  const PreStart* st = (const PreStart*)lds;
+  if constexpr (PLANNED) {
+    st = (const PreStart*)p.ws_plan + b;
+    if (uni(st->u) < 0) return;
+  } else {
+    if (!prefill_start<PR>(p, b, (PreStart*)lds, (int64_t*)(lds + sizeof(PreStart)))) return;
+  }
+  const int64_t C = uni64(st->C);
+  const int NUa = (int)active_units(C, p.NUP);
+  const int u = uni(st->u);
+  int kvh = uni(st->kvh);
+  int t = uni(st->t);
+  int seq = uni(st->seq);
   SeqView sv;
-  sv.q_len = uni(rec[6]);
-  sv.kv_total = uni(rec[7]);
-  sv.qs = uni64(pair(8));
-  sv.ctx = uni64(pair(10));
-  int64_t x = uni64(pair(12));
-  const int64_t x1 = uni64(pair(14));
+  sv.q_len = uni(st->q_len);
+  sv.kv_total = uni(st->kv_total);
+  sv.qs = uni64(st->qs);
+  sv.ctx = uni64(st->ctx);
+  int64_t x = uni64(st->x0);
+  const int64_t x1 = uni64(st->x1);
   const int total = (int)(x1 - x);  // positions of this unit: < 2^31 (C / NUa + 1)
   int R = sv.q_len * p.G;
   int tiles = (R + p.PR - 1) / p.PR;
@@ -2281,16 +2300,17 @@ __device__ __forceinline__ void prefill_units(const PAParams& p, TileFn&& tile) 
   // chunks max(0, a - kTileCost) .. max(0, b - kTileCost) - 1, the same map at both ends
   // of every unit, so the pieces partition the chunks; a range inside the virtual prefix is
   // empty and skipped.
-  int64_t a = rem;
+  int64_t a = uni(st->rem);
+  if constexpr (!PLANNED) __syncthreads();  // every wave has read the start before the tile's loads overwrite it
   bool first = true;
   for (;;) {
     const int64_t tw = kTileCost + n_t;
-    const int64_t b = min(tw, a + (x1 - x));
-    const int c_lo = (int)max((int64_t)0, a - kTileCost), c_hi = (int)max((int64_t)0, b - kTileCost);
+    const int64_t e = min(tw, a + (x1 - x));
+    const int c_lo = (int)max((int64_t)0, a - kTileCost), c_hi = (int)max((int64_t)0, e - kTileCost);
     if (c_hi > c_lo) {
       const bool whole = c_lo == 0 && c_hi == n_t;
       const int64_t slot = 2 * (int64_t)u + (first ? 0 : 1);
-      const int rest = (int)(x1 - (x + (b - a)));
+      const int rest = (int)(x1 - (x + (e - a)));
       tile(sv, R, seq, kvh, t, c_lo, c_hi, !whole, slot, rest, total);
       if (threadIdx.x == 0 && c_lo == 0 && c_hi < n_t) {
         // the tile continues in units u + 1 .. u1, each holding it as its first piece
@@ -2300,15 +2320,15 @@ __device__ __forceinline__ void prefill_units(const PAParams& p, TileFn&& tile) 
       }
       first = false;
     }
-    x += b - a;
+    x += e - a;
     if (x >= x1) break;
     a = 0;
     if (++t == tiles) {
       t = 0;
       if (++kvh == p.Hkv) {
         kvh = 0;
-        if (++k >= n_pre) return;  // cannot happen: the flat space ends with the last sequence
-        seq = uni(p.ws_pre_list[k]);
+        seq = uni(next_prefill_seq(p, seq + 1));
+        if (seq >= p.B) return;  // cannot happen: the flat space ends with the last sequence
         sv = seq_view_uniform(p, seq);
         R = sv.q_len * p.G;
         tiles = (R + p.PR - 1) / p.PR;
@@ -2318,19 +2338,44 @@ __device__ __forceinline__ void prefill_units(const PAParams& p, TileFn&& tile) 
   }
 }
 
-// 4-wave workgroups of 64 NT rows (PAParams::PR), 2 per CU.
-template <class E, int D, bool KV8>
-__global__ __launch_bounds__(256, 2) void pa_prefill_kernel(PAParams p) {
-  using L = PrefillLds<D>;
-  __shared__ __attribute__((aligned(1024))) char lds[(KV8 ? 2 : L::kStages) * L::kStageBytes];
+// LDS of a prefill workgroup: the ring's stages (3 over 16-bit caches, 2 over E4M3 caches).
+template <int D, bool KV8>
+constexpr int prefill_lds_bytes() {
+  return (KV8 ? 2 : PrefillLds<D>::kStages) * PrefillLds<D>::kStageBytes;
+}
+
+template <class E, int D, bool KV8, bool PLANNED>
+__device__ __forceinline__ void prefill_unit(const PAParams& p, int block, char* lds) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  prefill_units(p, [&](const SeqView& sv, int R, int seq, int kvh, int t, int c_lo, int c_hi, bool partial,
-                       int64_t slot, int rest, int total) {
+  prefill_units<kWavesPerWG * 16 * prefill_nt<KV8>(), PLANNED>(p, block, lds, [&](const SeqView& sv, int R, int seq, int kvh, int t, int c_lo, int c_hi, bool partial,
+                                   int64_t slot, int rest, int total) {
     if constexpr (KV8)
       prefill_tile_kv8<E, D>(lds, p, sv, R, seq, kvh, t, c_lo, c_hi, w, partial, slot, rest, total);
     else
       prefill_tile<E, D>(lds, p, sv, R, seq, kvh, t, c_lo, c_hi, w, partial, slot, rest, total);
   });
+}
+
+// 4-wave workgroups of 64 NT rows (PAParams::PR), 2 per CU.
+template <class E, int D, bool KV8>
+__global__ __launch_bounds__(256, 2) void pa_prefill_kernel(PAParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[prefill_lds_bytes<D, KV8>()];
+  prefill_unit<E, D, KV8, true>(p, blockIdx.x, lds);
+}
+
+// A mixed batch in one launch: the first ND workgroups are its decode units, the next NUP its
+// prefill units, which find their own starts. For batches whose decode part is small or empty
+// (launch_mixed): its workgroups leave their places at once, and no launch runs ahead of the
+// prefill work. Four prompts of 300-2500 tokens (D = 128, bf16): step 201 -> 176 us; two chunks
+// of 900-1024 tokens over 4000-10000 cached ones, E4M3: 328 -> 310 us.
+template <class E, int D, bool KV8>
+__global__ __launch_bounds__(256, 2) void pa_mixed_kernel(PAParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[prefill_lds_bytes<D, KV8>()];
+  const int b = blockIdx.x;
+  if (b < p.ND)
+    decode_unit<E, D, 1, KV8, 1>(p, b);
+  else
+    prefill_unit<E, D, KV8, false>(p, b - p.ND, lds);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2365,13 +2410,10 @@ static int resident_blocks(const void* kernel, int block_threads = 256, int* per
   return blocks;
 }
 
-template <class E, int D, int NT, bool KV8, int NX = 1>
-static int launch_decode_nt(PAParams& p, hipStream_t s) {
-  const void* k = (const void*)&pa_decode_kernel<E, D, NT, KV8, NX>;
-  const int plan_wgs = p.PLAN ? 1 : 0;  // workgroup 0 plans the prefill launch
-  int per_cu = 1;
-  const int resident = resident_blocks(k, 256, &per_cu);
-  int waves = (resident - plan_wgs) * kWavesPerWG;
+// Sets the decode units (PAParams::NU, R1) of a launch of `kernel`, which holds `resident`
+// workgroups, `per_cu` on each CU; returns their workgroups.
+static int decode_units(PAParams& p, int resident, int per_cu, bool kv8) {
+  int waves = resident * kWavesPerWG;
   if (waves > kMaxDecodeWaves) waves = kMaxDecodeWaves;
   int64_t units = waves / p.HGW;
   // 16-bit caches: half the resident waves. Each split segment leaves one fp32 partial per
@@ -2388,7 +2430,7 @@ static int launch_decode_nt(PAParams& p, hipStream_t s) {
   // (the 64-row cascade tiles, 48 or 64 verify rows) keeps them all: halving would idle half
   // the CUs.
   if (per_cu >= 2) {
-    if (!KV8)
+    if (!kv8)
       units /= 2;
     else if (per_cu >= 3)
       units = units * 2 / 3;
@@ -2405,12 +2447,75 @@ static int launch_decode_nt(PAParams& p, hipStream_t s) {
   p.NU = (int32_t)units;
   const int wgs = (p.NU * p.HGW + kWavesPerWG - 1) / kWavesPerWG;
   // units whose last workgroup is dispatched before every CU holds one (unit u's waves are
-  // u HGW .. (u + 1) HGW - 1, behind the planning workgroup)
+  // u HGW .. (u + 1) HGW - 1)
   const int cus = per_cu > 0 ? resident / per_cu : resident;
-  const int64_t r1 = (int64_t)kWavesPerWG * (cus - plan_wgs) / p.HGW;
-  p.R1 = (int32_t)(wgs + plan_wgs > cus ? (r1 < 0 ? 0 : (r1 < units ? r1 : units)) : units);
-  hipLaunchKernelGGL((pa_decode_kernel<E, D, NT, KV8, NX>), dim3(wgs + plan_wgs), dim3(256), 0, s, p);
+  const int64_t r1 = (int64_t)kWavesPerWG * cus / p.HGW;
+  p.R1 = (int32_t)(wgs > cus && r1 < units ? r1 : units);
+  return wgs;
+}
+
+template <class E, int D, int NT, bool KV8, int NX = 1>
+static int launch_decode_nt(PAParams& p, hipStream_t s) {
+  int per_cu = 1;
+  const int resident = resident_blocks((const void*)&pa_decode_kernel<E, D, NT, KV8, NX>, 256, &per_cu);
+  const int wgs = decode_units(p, resident, per_cu, KV8);
+  p.ND = p.NUP > 0 ? wgs : 0;  // NUP > 0: the workgroups behind the decode units plan the prefill launch
+  hipLaunchKernelGGL((pa_decode_kernel<E, D, NT, KV8, NX>), dim3(wgs + p.NUP), dim3(256), 0, s, p);
   return (int)hipGetLastError();
+}
+
+// The decode launch of a batch whose decode-class sequences take NT 16-row tiles (no cascade).
+template <class E, int D, bool KV8>
+static int launch_decode(PAParams& p, int NT, hipStream_t s) {
+  switch (NT) {
+    case 1: return launch_decode_nt<E, D, 1, KV8>(p, s);
+    case 2: return launch_decode_nt<E, D, 2, KV8>(p, s);
+    case 3: return launch_decode_nt<E, D, 3, KV8>(p, s);
+    case 4: return launch_decode_nt<E, D, 4, KV8>(p, s);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+
+// Decode chunks per unit up to which a mixed batch takes one launch (launch_mixed).
+constexpr int64_t kFusedUnitChunks = 4;
+
+// A batch with prefill-class sequences. Where the static shape leaves the decode part at most
+// kFusedUnitChunks chunks per unit (prompts alone, or with a few short decodes), decode and
+// prefill units share one launch. A larger decode part goes ahead in a launch of its own: the
+// two kinds of workgroup on one CU take longer together than one after the other (512 decodes
+// of 255-4095 keys beside four 384-token chunks 851 us in one launch, 816 apart; 100 decodes of
+// 255-2000 keys beside the same chunks 216 and 188; 512 decodes beside one 17-token chunk 721
+// and 741). Apart as well when the call's kernels are being timed, or when a decode row needs more
+// than one 16-row tile (GQA groups above 16).
+template <class E, int D, bool KV8>
+static int launch_mixed(PAParams& p, int NT, int32_t max_q, hipStream_t s, LaunchLog& log) {
+  p.PR = kWavesPerWG * 16 * prefill_nt<KV8>();
+  // units x 2 partial slots x tile rows stay within the workspace's kMaxPrefillUnits x 2 x kPrefillRows
+  const int cap = kMaxPrefillUnits * kPrefillRows / p.PR;
+  // sequences that can be decode class: each of the others takes at most max_q of the T tokens
+  const int64_t over = p.T - (int64_t)p.B * p.QS;
+  const int64_t n_pre = over > 0 ? (over + max_q - p.QS - 1) / (max_q - p.QS) : 0;
+  const int64_t n_dec = p.B > n_pre ? p.B - n_pre : 0;
+  const int64_t dec_chunks = n_dec * (p.Hkv / p.HGW) * (((int64_t)p.W * p.BS + kChunk - 1) / kChunk);
+  int err, per_cu = 1;
+  const int resident = resident_blocks((const void*)&pa_mixed_kernel<E, D, KV8>, 256, &per_cu);
+  const int wgs = decode_units(p, resident, per_cu, KV8);
+  if (log.events || NT > 1 || dec_chunks > kFusedUnitChunks * p.NU) {
+    p.NUP = std::max(8, std::min(resident_blocks((const void*)&pa_prefill_kernel<E, D, KV8>), cap) / 8 * 8);
+    if ((err = launch_decode<E, D, KV8>(p, NT, s))) return err;
+    log.after_launch(1, s);
+    hipLaunchKernelGGL((pa_prefill_kernel<E, D, KV8>), dim3(p.NUP), dim3(256), 0, s, p);
+    if ((err = (int)hipGetLastError())) return err;
+    log.after_launch(2, s);
+    return 0;
+  }
+  p.NUP = std::max(8, std::min(resident, cap) / 8 * 8);
+  p.ND = (wgs + 7) / 8 * 8;  // prefill workgroup b keeps XCD b % 8
+  hipLaunchKernelGGL((pa_mixed_kernel<E, D, KV8>), dim3(p.ND + p.NUP), dim3(256), 0, s, p);
+  if ((err = (int)hipGetLastError())) return err;
+  log.after_launch(1, s);
+  log.after_launch(2, s);
+  return 0;
 }
 
 template <class E, int D, bool KV8>
@@ -2422,7 +2527,6 @@ static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipSt
     log.after_launch(1, s);
     return 0;
   }
-  p.PLAN = plan.launch_prefill ? 1 : 0;
   p.CASC = plan.cascade ? 1 : 0;
   if (plan.cascade) {
     hipLaunchKernelGGL(pa_share_kernel, dim3(1), dim3(kPlanThreads), 0, s, p);
@@ -2430,41 +2534,13 @@ static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipSt
     log.after_launch(5, s);
   }
   if (plan.launch_prefill) {
-    // the unit count is fixed before the decode launch: both kernels write merge jobs. Units x
-    // 2 partial slots x tile rows stay within the workspace's kMaxPrefillUnits x 2 x kPrefillRows.
-    p.PR = kWavesPerWG * 16 * prefill_nt<KV8>();
-    int units = resident_blocks((const void*)&pa_prefill_kernel<E, D, KV8>);
-    const int cap = kMaxPrefillUnits * kPrefillRows / p.PR;
-    if (units > cap) units = cap;
-    p.NUP = units / 8 * 8;
-    if (p.NUP < 8) p.NUP = 8;
-  }
-  switch (plan.NT) {
-    case 1:
-      if constexpr (!KV8) {
-        if (plan.cascade && p.XR == 64) {  // 64-row prefix groups (16-bit caches)
-          err = launch_decode_nt<E, D, 1, KV8, 4>(p, s);
-          break;
-        }
-      } else {
-        if (plan.cascade && p.XR == 32) {  // 32-row prefix groups (E4M3 caches)
-          err = launch_decode_nt<E, D, 1, KV8, 2>(p, s);
-          break;
-        }
-      }
-      err = launch_decode_nt<E, D, 1, KV8>(p, s);
-      break;
-    case 2: err = launch_decode_nt<E, D, 2, KV8>(p, s); break;
-    case 3: err = launch_decode_nt<E, D, 3, KV8>(p, s); break;
-    case 4: err = launch_decode_nt<E, D, 4, KV8>(p, s); break;
-    default: return (int)hipErrorInvalidValue;
-  }
-  if (err) return err;
-  log.after_launch(1, s);
-  if (plan.launch_prefill) {
-    hipLaunchKernelGGL((pa_prefill_kernel<E, D, KV8>), dim3(p.NUP), dim3(256), 0, s, p);
-    if ((err = (int)hipGetLastError())) return err;
-    log.after_launch(2, s);
+    if ((err = launch_mixed<E, D, KV8>(p, plan.NT, max_q, s, log))) return err;
+  } else {
+    constexpr int NX = KV8 ? 2 : 4;  // 64-row prefix groups (32 over E4M3 caches)
+    err = plan.cascade && p.XR == 16 * NX ? launch_decode_nt<E, D, 1, KV8, NX>(p, s)
+                                          : launch_decode<E, D, KV8>(p, plan.NT, s);
+    if (err) return err;
+    log.after_launch(1, s);
   }
   const int mr = plan.launch_prefill ? merge_rows_decode<D, true>() : merge_rows_decode<D, false>();
   const int cd = (p.HGW * p.RS + mr - 1) / mr;
