@@ -13,8 +13,11 @@
 //   gemv + silu_mul (GLU): the gate_up projection with silu_mul in its epilogue: a wave
 //                takes gate rows j .. and the up rows I + j .., rounds both sums to the
 //                storage type (the projection's output) and applies silu_mul's arithmetic.
+#include <type_traits>
+
 #include "kvh_device.h"
 #include "kvh_internal.h"
+#include "skinny.h"
 
 namespace kvh {
 namespace {
@@ -286,80 +289,59 @@ int launch_gemv_t(const void* x, int64_t x_rs, const void* w, int64_t w_rs, void
   }
 }
 
-// Skinny GEMM for 5 .. 64 rows: y[m][n] = sum_k x[m][k] w[n][k] on v_mfma_f32_16x16x32. A
-// workgroup of 8 waves owns 16 weight rows (one MFMA A tile, n0 .. n0 + 15); wave w takes the
-// k-slice [w K / 8, (w + 1) K / 8) in 32-wide steps, four in flight, with MT = ceil(m / 16)
-// B tiles of x (rows past m read row m - 1 and are dropped). The 8 partial 16 x 16 MT tiles
-// meet in LDS and are summed in wave order (deterministic) and rounded once. Lane l of a tile
-// holds D[4 (l / 16) + r][l % 16], r < 4: weight row n0 + 4 (l / 16) + r, x row 16 mt + l % 16.
-// GLU: the workgroup owns output columns c0 .. c0 + 7 (c0 = 8 blockIdx) of silu_mul(gate_up):
-// A rows i < 8 are gate rows c0 + i, rows i >= 8 the up rows inter + c0 + i - 8; the epilogue
-// rounds each sum to the storage type and applies silu_mul's arithmetic (the bits of the plain
-// kernel followed by kvh_silu_mul). n is then the intermediate size.
-constexpr int kSkinnyWaves = 8;
-
-template <class E, int MT, bool GLU = false>
-__global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const uint16_t* __restrict__ x,
-                                                                        int64_t x_rs,
-                                                                        const uint16_t* __restrict__ w,
-                                                                        int64_t w_rs, uint16_t* __restrict__ y,
-                                                                        int64_t y_rs, int m, int k, int n) {
-  __shared__ f32x4 red[kSkinnyWaves][MT][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 15, j = lane >> 4;
-  const int64_t n0 = (int64_t)blockIdx.x * (GLU ? 8 : 16);
-  const int slice = k / kSkinnyWaves;
-  const int k_lo = wave * slice;
-  const int64_t wrow = GLU ? (i < 8 ? n0 + i : n + n0 + i - 8) : n0 + i;
-  const uint16_t* wr = w + wrow * w_rs + k_lo + 8 * j;
-  const uint16_t* xr[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) xr[t] = x + (int64_t)min(16 * t + i, m - 1) * x_rs + k_lo + 8 * j;
+// Skinny GEMM for up to 64 rows: y[m][n] = sum_k x[m][k] w[n][k] on v_mfma_f32_16x16x32, in the
+// forms of skinny.h. `ks` waves share a tile of TR = 16 or 8 weight rows, each a k-slice, with MT
+// B tiles of TR rows of x (rows past m are dropped). The partial tiles meet in LDS and are summed
+// in slice order (deterministic) and rounded once. Lane l of a tile holds D[4 (l / 16) + r][l %
+// 16], r < 4: weight row n0 + 4 (l / 16) + r, x row TR mt + l % 16.
+// GLU: a tile gives TR / 2 output columns c0 .. of silu_mul(gate_up): its first TR / 2 rows are
+// gate rows c0 + i, the others the up rows inter + c0 + i; the epilogue rounds each sum to the
+// storage type and applies silu_mul's arithmetic (the bits of the plain kernel followed by
+// kvh_silu_mul). n is then the intermediate size.
+template <class E, SkinnyForm F, int MT, bool GLU>
+__global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_rs,
+                                                                        const uint16_t* __restrict__ w, int64_t w_rs,
+                                                                        uint16_t* __restrict__ y, int64_t y_rs, int m,
+                                                                        int k, int n, int ks, int vec) {
+  constexpr int THREADS = 64 * kSkinnyWaves;
+  constexpr int TR = skinny_rows(F), COLS = GLU ? TR / 2 : TR;  // weight rows and outputs of a tile
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  f32x4(*red)[MT][64] = (f32x4(*)[MT][64])lds;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = skinny_row<F>(lane);
+  const int tiles = kSkinnyWaves / ks;  // of this workgroup
+  const int64_t tile0 = (int64_t)blockIdx.x * tiles, all = n / COLS;
+  const int64_t n0 = min(tile0 + wave / ks, all - 1) * COLS;  // waves past the last tile repeat it
+  const int slice = wave % ks, len = k / ks;
+  const int64_t wrow = GLU ? (i < COLS ? n0 + i : n + n0 + i - COLS) : n0 + i;
+  const uint16_t* wr = w + wrow * w_rs + slice * len + skinny_k<F>(lane);
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int kk = 0; kk < slice; kk += 128) {
-    u32x4 a[4], b[4][MT];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      a[u] = *(const u32x4*)(wr + kk + 32 * u);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) b[u][t] = *(const u32x4*)(xr[t] + kk + 32 * u);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) acc[t] = E::mfma(a[u], b[u][t], acc[t]);
-  }
+  skinny_slice<E, F, MT>(wr, x, x_rs, m, ks, slice, len, lds, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
-  if constexpr (GLU) {
-    // 8 x 16 MT outputs; thread q: column c = q % 8 of x row 16 t + (q / 8) % 16, t = q / 128;
-    // the gate sum is D[c][.] (lane 16 (c / 4) + row, element c % 4), the up sum D[8 + c][.]
-    for (int q = threadIdx.x; q < MT * 128; q += 64 * kSkinnyWaves) {
-      const int t = q >> 7, mr = (q >> 3) & 15, c = q & 7;
-      const int row = 16 * t + mr;
-      if (row >= m) continue;
-      const int lg = 16 * (c >> 2) + mr, lu = 16 * (2 + (c >> 2)) + mr, r = c & 3;
-      float g = 0.f, u = 0.f;
+  // thread q: 4 outputs of one x row, those of lane l = 16 jj + c of B tile t (GLU: their up sums
+  // lie TR / 2 rows, 16 (COLS / 4) lanes, further on)
+  constexpr int L = TR * (COLS / 4);
+  for (int q = threadIdx.x; q < tiles * MT * L; q += THREADS) {
+    const int c = q % TR, jj = q / TR % (COLS / 4), t = q / L % MT, tt = q / (L * MT);
+    const int row = TR * t + c, l = 16 * jj + c;
+    if (row >= m || tile0 + tt >= all) continue;
+    f32x4 o = skinny_sum<F, MT>(red + tt * ks, ks, t, l);
+    if constexpr (GLU) {
+      const f32x4 up = skinny_sum<F, MT>(red + tt * ks, ks, t, l + 4 * COLS);
 #pragma unroll
-      for (int v = 0; v < kSkinnyWaves; ++v) {
-        g += red[v][t][lg][r];
-        u += red[v][t][lu][r];
-      }
-      y[row * y_rs + n0 + c] = (uint16_t)(E::pack2(silu_mul1<E>(g, u), 0.f) & 0xffffu);
+      for (int r = 0; r < 4; ++r) o[r] = silu_mul1<E>(o[r], up[r]);
     }
-  } else {
-    // 16 x 16 MT outputs; thread q sums element q % 4 of lane (q / 4) % 64 of tile q / 256
-    for (int q = threadIdx.x; q < MT * 256; q += 64 * kSkinnyWaves) {
-      const int t = q >> 8, l = (q >> 2) & 63, r = q & 3;
-      const int row = 16 * t + (l & 15);
-      if (row >= m) continue;
-      float sum = 0.f;
+    uint16_t* dst = y + row * y_rs + (tile0 + tt) * COLS + 4 * jj;
+    const u32x2 packed = {E::pack2(o[0], o[1]), E::pack2(o[2], o[3])};
+    if (vec) {
+      *(u32x2*)dst = packed;
+    } else {
 #pragma unroll
-      for (int v = 0; v < kSkinnyWaves; ++v) sum += red[v][t][l][r];
-      y[row * y_rs + n0 + 4 * (l >> 4) + r] = (uint16_t)(E::pack2(sum, 0.f) & 0xffffu);
+      for (int r = 0; r < 4; ++r) dst[r] = (uint16_t)(packed[r / 2] >> (16 * (r & 1)));
     }
   }
 }
@@ -367,16 +349,32 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const ui
 template <class E, bool GLU>
 int launch_skinny_t(const void* x, int64_t x_rs, const void* w, int64_t w_rs, void* y, int64_t y_rs, int m, int n,
                     int k, hipStream_t s) {
-  const dim3 grid((unsigned)(n / (GLU ? 8 : 16))), block(64 * kSkinnyWaves);
-  const auto* xp = (const uint16_t*)x;
-  const auto* wp = (const uint16_t*)w;
-  auto* yp = (uint16_t*)y;
-  switch ((m + 15) / 16) {
-    case 1: hipLaunchKernelGGL((skinny_gemm_kernel<E, 1, GLU>), grid, block, 0, s, xp, x_rs, wp, w_rs, yp, y_rs, m, k, n); break;
-    case 2: hipLaunchKernelGGL((skinny_gemm_kernel<E, 2, GLU>), grid, block, 0, s, xp, x_rs, wp, w_rs, yp, y_rs, m, k, n); break;
-    case 3: hipLaunchKernelGGL((skinny_gemm_kernel<E, 3, GLU>), grid, block, 0, s, xp, x_rs, wp, w_rs, yp, y_rs, m, k, n); break;
-    default: hipLaunchKernelGGL((skinny_gemm_kernel<E, 4, GLU>), grid, block, 0, s, xp, x_rs, wp, w_rs, yp, y_rs, m, k, n); break;
+  const int64_t rows = GLU ? 2 * (int64_t)n : n;
+  const int ks = skinny_slices(rows, k, m), per = kSkinnyWaves / ks;
+  const int tiles = (int)(rows / skinny_rows(skinny_form(rows, m)));
+  const dim3 grid((unsigned)((tiles + per - 1) / per)), block(64 * kSkinnyWaves);
+  const int vec = (((uintptr_t)y | (uintptr_t)(2 * y_rs)) & 7) == 0;  // 8-byte stores
+#define KVH_LAUNCH_SKINNY(F, MT)                                                                                    \
+  hipLaunchKernelGGL((skinny_gemm_kernel<E, F, MT, GLU>), grid, block, (skinny_lds_bytes<F, MT>(ks)), s,             \
+                     (const uint16_t*)x, x_rs, (const uint16_t*)w, w_rs, (uint16_t*)y, y_rs, m, k, n, ks, vec)
+  switch (skinny_form(rows, m)) {
+    case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
+    case kSkinnyFull:
+      switch ((m + 15) / 16) {
+        case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1); break;
+        case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2); break;
+        case 3: KVH_LAUNCH_SKINNY(kSkinnyFull, 3); break;
+        default: KVH_LAUNCH_SKINNY(kSkinnyFull, 4); break;
+      }
+      break;
+    default:  // shared x: 8, 16, 32 or 64 rows
+      if (m <= 8) KVH_LAUNCH_SKINNY(kSkinnyShared, 1);
+      else if (m <= 16) KVH_LAUNCH_SKINNY(kSkinnyShared, 2);
+      else if (m <= 32) KVH_LAUNCH_SKINNY(kSkinnyShared, 4);
+      else KVH_LAUNCH_SKINNY(kSkinnyShared, 8);
+      break;
   }
+#undef KVH_LAUNCH_SKINNY
   return (int)hipGetLastError();
 }
 

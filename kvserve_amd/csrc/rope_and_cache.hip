@@ -21,6 +21,7 @@
 
 #include "kvh_device.h"
 #include "kvh_internal.h"
+#include "skinny.h"
 
 namespace kvh {
 
@@ -310,71 +311,75 @@ __global__ __launch_bounds__(256) void gemv_rope_cache_kernel(GemvRopeArgs a) {
   for (int m = 0; m < M; ++m) rope_pair_out<DT, KV8>(a, m, h, d, acc[m][0], acc[m][1]);
 }
 
-// The same for 5 .. 64 rows on the MFMA units, laid out as the skinny GEMM (engine_ops.hip):
-// a workgroup of 8 waves (k-slices) owns 8 pairs (one 16-row A tile: rows h D + d0 + i for
-// i < 8, h D + d0 + D / 2 + i - 8 for i >= 8) and MT = ceil(m / 16) B tiles of x; the eight
-// partial tiles meet in LDS, are summed in wave order and go through rope_pair_out.
-template <int DT, int MT, bool KV8>
-__global__ __launch_bounds__(512) void skinny_rope_cache_kernel(GemvRopeArgs a, int m) {
+// The same for 5 .. 64 rows on the MFMA units, laid out as the skinny GEMM (skinny.h,
+// engine_ops.hip): `ks` waves (k-slices) own NP = 8 or 4 pairs, one A tile of rows h D + d0 + i for
+// i < NP, h D + d0 + D / 2 + i - NP for i >= NP, and MT B tiles of x; the partial tiles meet in LDS,
+// are summed in slice order and go through rope_pair_out.
+template <int DT, SkinnyForm F, int MT, bool KV8>
+__global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(GemvRopeArgs a, int m, int ks) {
   using E = std::conditional_t<DT == 2, BF16, F16>;
-  __shared__ f32x4 red[8][MT][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 15, jg = lane >> 4;
+  constexpr int THREADS = 64 * kSkinnyWaves, TR = skinny_rows(F), NP = TR / 2;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  f32x4(*red)[MT][64] = (f32x4(*)[MT][64])lds;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = skinny_row<F>(lane);
   const int half = a.D / 2;
-  const int p0 = blockIdx.x * 8;  // first pair
+  const int tiles = kSkinnyWaves / ks;  // of this workgroup
+  const int tile0 = blockIdx.x * tiles, all = (a.H + 2 * a.Hkv) * half / NP;
+  const int p0 = min(tile0 + wave / ks, all - 1) * NP;  // first pair; waves past the last tile repeat it
   const int h = p0 / half, d0 = p0 % half;
-  const int64_t wrow = (int64_t)h * a.D + d0 + (i < 8 ? i : half + i - 8);
-  const int slice = a.k / 8;
-  const int k_lo = wave * slice;
-  const uint16_t* wr = a.w + wrow * a.w_rs + k_lo + 8 * jg;
-  const uint16_t* xr[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) xr[t] = a.x + (int64_t)min(16 * t + i, m - 1) * a.x_rs + k_lo + 8 * jg;
+  const int64_t wrow = (int64_t)h * a.D + d0 + (i < NP ? i : half + i - NP);
+  const int slice = wave % ks, len = a.k / ks;
+  const uint16_t* wr = a.w + wrow * a.w_rs + slice * len + skinny_k<F>(lane);
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int kk = 0; kk < slice; kk += 128) {
-    u32x4 av[4], bv[4][MT];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      av[u] = *(const u32x4*)(wr + kk + 32 * u);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) bv[u][t] = *(const u32x4*)(xr[t] + kk + 32 * u);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) acc[t] = E::mfma(av[u], bv[u][t], acc[t]);
-  }
+  skinny_slice<E, F, MT>(wr, a.x, a.x_rs, m, ks, slice, len, lds, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
-  for (int q = threadIdx.x; q < MT * 128; q += 512) {
-    const int t = q >> 7, mr = (q >> 3) & 15, c = q & 7;
-    const int row = 16 * t + mr;
-    if (row >= m) continue;
-    const int ll = 16 * (c >> 2) + mr, lh = 16 * (2 + (c >> 2)) + mr, r = c & 3;
-    float s_lo = 0.f, s_hi = 0.f;
+  // thread q: pairs 4 jj .. 4 jj + 3 of one x row; their second rows lie NP rows further on
+  constexpr int L = TR * (NP / 4);
+  for (int q = threadIdx.x; q < tiles * MT * L; q += THREADS) {
+    const int c = q % TR, jj = q / TR % (NP / 4), t = q / L % MT, tt = q / (L * MT);
+    const int row = TR * t + c, l = 16 * jj + c;
+    if (row >= m || tile0 + tt >= all) continue;
+    const f32x4 lo = skinny_sum<F, MT>(red + tt * ks, ks, t, l);
+    const f32x4 hi = skinny_sum<F, MT>(red + tt * ks, ks, t, l + 4 * NP);
+    const int pq = (tile0 + tt) * NP;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      s_lo += red[v][t][ll][r];
-      s_hi += red[v][t][lh][r];
-    }
-    rope_pair_out<DT, KV8>(a, row, h, d0 + c, s_lo, s_hi);
+    for (int r = 0; r < 4; ++r) rope_pair_out<DT, KV8>(a, row, pq / half, pq % half + 4 * jj + r, lo[r], hi[r]);
   }
 }
 
 template <int DT, bool KV8>
 static int launch_gemv_rope_dt(const GemvRopeArgs& a, int m, hipStream_t s) {
   const int waves = (a.H + 2 * a.Hkv) * (a.D / 2);
-  if (m > 4) {  // the skinny form: one workgroup per 8 pairs
-    const dim3 g2((unsigned)(waves / 8)), b2(512);
-    switch ((m + 15) / 16) {
-      case 1: hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, 1, KV8>), g2, b2, 0, s, a, m); break;
-      case 2: hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, 2, KV8>), g2, b2, 0, s, a, m); break;
-      case 3: hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, 3, KV8>), g2, b2, 0, s, a, m); break;
-      default: hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, 4, KV8>), g2, b2, 0, s, a, m); break;
+  if (m > 4) {  // the skinny form
+    const int64_t rows = 2 * (int64_t)waves;
+    const int ks = skinny_slices(rows, a.k, m), per = kSkinnyWaves / ks;
+    const int tiles = (int)(rows / skinny_rows(skinny_form(rows, m)));
+    const dim3 g2((unsigned)((tiles + per - 1) / per)), b2(64 * kSkinnyWaves);
+#define KVH_LAUNCH_SKINNY(F, MT) \
+  hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, F, MT, KV8>), g2, b2, (skinny_lds_bytes<F, MT>(ks)), s, a, m, ks)
+    switch (skinny_form(rows, m)) {
+      case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
+      case kSkinnyFull:
+        switch ((m + 15) / 16) {
+          case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1); break;
+          case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2); break;
+          case 3: KVH_LAUNCH_SKINNY(kSkinnyFull, 3); break;
+          default: KVH_LAUNCH_SKINNY(kSkinnyFull, 4); break;
+        }
+        break;
+      default:  // shared x: 8, 16, 32 or 64 rows
+        if (m <= 8) KVH_LAUNCH_SKINNY(kSkinnyShared, 1);
+        else if (m <= 16) KVH_LAUNCH_SKINNY(kSkinnyShared, 2);
+        else if (m <= 32) KVH_LAUNCH_SKINNY(kSkinnyShared, 4);
+        else KVH_LAUNCH_SKINNY(kSkinnyShared, 8);
+        break;
     }
+#undef KVH_LAUNCH_SKINNY
     return (int)hipGetLastError();
   }
   const dim3 grid((waves + 3) / 4);

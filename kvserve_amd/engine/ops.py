@@ -59,18 +59,32 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 
 def skinny_wins(m: int, n: int, k: int) -> bool:
-    """Where kvh_gemm_skinny beats hipBLASLt inside the decode graph (measured on MI355X at the
-    1B / 8B shapes; the skinny kernel re-reads x per 16 weight rows, so its edge shrinks with m
-    and the weight size): up to 8 rows for weights up to 80 MB (8B o_proj 9.7 vs 19.3 us
-    alone; decode at batch 8: 8B +3%, 1B +7%), up to 32 rows for weights up to 13 MB (the 1B
-    QKV and o_proj; 1B at batch 32 +4%). Larger weights at 16 rows, everything at 64 rows and
-    the 8B o_proj at 32 won alone but not inside the model."""
+    """Where kvh_gemm_skinny beats hipBLASLt, by weight shape (n, k), cold weights on MI355X, bf16
+    (skinny / hipBLASLt in us):
+      up to 8 rows    weights of 8192 rows or more ((28672, 4096) 44 / 62, (128256, 2048) 96 / 117,
+                      (128256, 4096) 178 / 191, (16384, 2048) 16 / 18.8) and up to 40 MB ((2048,
+                      8192) 10 / 12.7, (4096, 4096) 10 / 15.5); not (4096, 14336) 28 / 26
+      up to 16 rows   the large ones (44 / 60, 101 / 128, 175 / 194, 16 / 17.4), up to 13 MB
+                      ((3072, 2048) 6.6 / 11.5) and 4096 rows up to 40 MB ((4096, 4096) 11 / 15.6);
+                      not (2048, 8192) 17 / 13.3
+      up to 32 rows   up to 13 MB ((3072, 2048) 8.5 / 11.7); not (128256, 4096) 212 / 203"""
     if n % 16 or k % 1024:
         return False
     w_bytes = 2 * n * k
     if m <= 8:
-        return w_bytes <= 80e6
+        return n >= 8192 or w_bytes <= 40e6
+    if m <= 16:
+        return n >= 8192 or w_bytes <= 13e6 or (n >= 4096 and w_bytes <= 40e6)
     return m <= 32 and w_bytes <= 13e6
+
+
+def mlp_act_fused(m: int, two_i: int, k: int) -> bool:
+    """Whether the gate_up projection of m rows takes kvh_gemm_skinny_silu_mul: where the skinny
+    GEMM wins, and up to 32 rows of weights of 8192 rows or more, where it is level with hipBLASLt
+    ((28672, 4096) 53 / 54 us, (16384, 2048) 17 / 17) and saves the activation's launch (5 us)."""
+    if two_i % 16 or k % 1024:
+        return False
+    return skinny_wins(m, two_i, k) or (m <= 32 and two_i >= 8192)
 
 
 def qkv_rope_fused(m: int, n: int, k: int) -> bool:
@@ -122,7 +136,7 @@ def mlp_act(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
     _same_gpu(x, gate_up_weight)
     if m > GEMV_MAX_ROWS:
         two_i, k = gate_up_weight.shape
-        if two_i % 16 or not skinny_wins(m, two_i, k):
+        if not mlp_act_fused(m, two_i, k):
             return silu_mul(linear(x, gate_up_weight))
         y = torch.empty((m, two_i // 2), dtype=x.dtype, device=x.device)
         st = _lib.load().kvh_gemm_skinny_silu_mul(x.data_ptr(), x.stride(0), gate_up_weight.data_ptr(),
