@@ -141,11 +141,39 @@ struct LaneOffsets {
   uint32_t v;  // (4j * v_ss + VW n) * 2
 };
 
-template <int D, bool KV8 = false>
+// Whole-line K reads (LINES), for up to 8 query rows (R <= 8, one tile): an instruction reads 128
+// bytes of 8 tokens instead of 64 bytes of 16. The A operand then holds 8 tokens twice, rows i and
+// i + 8 the same token at two neighbouring 16-byte chunks, and the B operand the query rows
+// likewise (lane column n: row n % 8, chunk n / 8), which takes the columns that 8 rows or fewer
+// leave idle anyway: S is the sum of the products of equal halves (line_scores), in as many MFMAs
+// as before. A non-temporal load does not keep the line's other half for the next instruction, so
+// half-line reads ask the L2 twice for every line. Rows of 128 bytes or more: 16-bit caches, and
+// E4M3 caches at D = 128.
+template <int D, bool KV8>
+constexpr bool can_read_lines() {
+  return !KV8 || D == 128;
+}
+constexpr int kLineRows = 8;
+// Where whole-line reads pay (bf16, times in us without / with):
+//  * the stream-K decode over E4M3 caches: 64 sequences of 1023-8191 keys, step 114.9 / 113.6; over
+//    16-bit caches only in units of up to kLineUnitChunks chunks: 16 sequences of 200-2200 keys 29.7 /
+//    28.5, but the 64 sequences (73 chunks a unit) 200.7 / 201.7, 512 sequences 801 / 811;
+//  * the short decode, together with non-temporal loads, from kShortLines = B Hkv D: 128 x 1000 keys
+//    102 / 88 (D = 128), 60 / 52 (D = 64), 32 x 1000 28.2 / 24.9, 16 x 500 12.4 / 11.3; below it the
+//    caches' half-line hits win (8 x 500 keys, D = 64: 7.3 / 8.5).
+constexpr int kLineUnitChunks = 32;
+constexpr int64_t kShortLines = 16384;
+
+template <int D, bool KV8 = false, bool LINES = false>
 __device__ __forceinline__ LaneOffsets lane_offsets(const PAParams& p) {
   const int lane = threadIdx.x & 63;
   const int j = lane >> 4, n = lane & 15;
   LaneOffsets o;
+  if (LINES) {  // token n % 8 of a group of 8, 16-byte chunk 2 j + n / 8 of the line
+    o.k = (uint32_t)((n & 7) * (uint32_t)p.k_ss) * (KV8 ? 1u : 2u) + 16u * (uint32_t)(2 * j + (n >> 3));
+    o.v = (uint32_t)(4 * j * (uint32_t)p.v_ss + (D / 16) * n) * (KV8 ? 1u : 2u);
+    return o;
+  }
   if (KV8) {  // one byte per element
     o.k = (uint32_t)(n * (uint32_t)p.k_ss + 16 * j);
     o.v = (uint32_t)(4 * j * (uint32_t)p.v_ss + (D / 16) * n);
@@ -172,15 +200,24 @@ __device__ __forceinline__ T stream_load(const void* p) {
 // Loads are unconditional so the chunk loop stays straight-line (no waits merged at
 // branch joins): an absent tile (blk < 0) reads block 0, which the API guarantees exists,
 // and is masked out of the scores and zeroed out of V like any invalid key.
-template <int D, bool NTL>
+// LINES: r.k[t][g D / 64 + cc] is line cc of the 8-token group g of tile t.
+template <int D, bool NTL, bool LINES>
 __device__ __forceinline__ void load_k(KRegs<D>& r, const PAParams& p, const ChunkRef& c, int kvh, uint32_t k_lane) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int64_t blk = c.blk[t] >= 0 ? c.blk[t] : 0;
     const int slot0 = (c.tok0 + 16 * t) % p.BS;
     const char* page = (const char*)p.kc + (blk * p.k_sb + (int64_t)kvh * p.k_sh + (int64_t)slot0 * p.k_ss) * 2;
+    if constexpr (LINES) {
 #pragma unroll
-    for (int cc = 0; cc < D / 32; ++cc) r.k[t][cc] = stream_load<u32x4, NTL>(page + k_lane + 64 * cc);
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int cc = 0; cc < D / 64; ++cc)
+          r.k[t][g * (D / 64) + cc] = stream_load<u32x4, NTL>(page + (int64_t)g * 16 * p.k_ss + k_lane + 128 * cc);
+    } else {
+#pragma unroll
+      for (int cc = 0; cc < D / 32; ++cc) r.k[t][cc] = stream_load<u32x4, NTL>(page + k_lane + 64 * cc);
+    }
   }
 }
 
@@ -210,15 +247,17 @@ __device__ __forceinline__ void load_v(VRegs<D>& r, const PAParams& p, const Chu
   }
 }
 
-template <int D, bool NTL>
+template <int D, bool NTL, bool LINES>
 __device__ __forceinline__ void load_k(KRegs8<D>& r, const PAParams& p, const ChunkRef& c, int kvh, uint32_t k_lane) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int64_t blk = c.blk[t] >= 0 ? c.blk[t] : 0;
     const int slot0 = (c.tok0 + 16 * t) % p.BS;
     const char* page = (const char*)p.kc + blk * p.k_sb + (int64_t)kvh * p.k_sh + (int64_t)slot0 * p.k_ss;
+    // LINES (D = 128): one line per token, group cc of the tile's two
 #pragma unroll
-    for (int cc = 0; cc < D / 64; ++cc) r.k[t][cc] = stream_load<u32x4, NTL>(page + k_lane + 64 * cc);
+    for (int cc = 0; cc < D / 64; ++cc)
+      r.k[t][cc] = stream_load<u32x4, NTL>(page + k_lane + (LINES ? (int64_t)cc * 8 * p.k_ss : (int64_t)64 * cc));
   }
 }
 
@@ -263,7 +302,9 @@ struct WaveState {
 };
 
 // Q rows of tile t: global row r = row0 + 16t + n, valid when r < R.
-template <int D, int NT, bool KV8 = false>
+// LINES: the operand's column n is row n % 8 at chunk n / 8 (see can_read_lines); D / 64 operands
+// are used (two over E4M3 caches), and columns 8 .. 15 see no key.
+template <int D, int NT, bool KV8 = false, bool LINES = false>
 __device__ __forceinline__ void load_q(WaveState<D, NT>& s, const PAParams& p, int64_t q_start, int R, int row0,
                                        int kvh, int64_t ctx, int64_t kv_total) {
   const int lane = threadIdx.x & 63;
@@ -278,6 +319,21 @@ __device__ __forceinline__ void load_q(WaveState<D, NT>& s, const PAParams& p, i
     s.nsh[t] = 0.f;
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) s.acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (LINES) {
+      static_assert(NT == 1, "whole-line reads serve one tile");
+      const int rr = n & 7, hb = n >> 3;
+      const bool in = rr < R;
+      const int qi = in ? rr / p.G : 0, g = in ? rr % p.G : 0;
+      const uint16_t* qp = q + (q_start + qi) * p.q_ts + (int64_t)(kvh * p.G + g) * p.q_hs;
+#pragma unroll
+      for (int c = 0; c < (KV8 ? 2 : D / 64); ++c) {
+        const u32x4 x = *(const u32x4*)(qp + (KV8 ? 32 * j + 16 * hb + 8 * c : 64 * c + 16 * j + 8 * hb));
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s.q[t][c][w] = in ? x[w] : 0u;
+      }
+      s.limit[t] = n < R ? (int)clamp64(ctx + qi + 1, 0, kv_total) : 0;
+      continue;
+    }
     if (r < R) {
       const int qi = r / p.G, g = r % p.G;
       const uint16_t* qp = q + (q_start + qi) * p.q_ts + (int64_t)(kvh * p.G + g) * p.q_hs;
@@ -296,17 +352,56 @@ __device__ __forceinline__ void load_q(WaveState<D, NT>& s, const PAParams& p, i
   }
 }
 
+// S^T of one tile from whole-line K operands (can_read_lines): groups 0 and 1 give two accumulators
+// whose valid quarters are rows and columns 0-7 (even chunks) and 8-15 (odd chunks). One swap puts
+// the first quarters of both groups into one register (lanes 0-31 group 0, 32-63 group 1) and the
+// second ones into another, which a rotation by 8 lanes brings under the first: lane (j, n) ends
+// up with token 4 j + e of the tile, as without LINES. Columns 8-15 hold sums of unequal halves;
+// their rows have no visible key.
+template <class E, int D, class KR>
+__device__ __forceinline__ f32x4 line_scores(const WaveState<D, 1>& s, const KR& kr, int tile) {
+  f32x4 x[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (std::is_same_v<KR, KRegs<D>>) {
+#pragma unroll
+      for (int cc = 0; cc < D / 64; ++cc) a = E::mfma(kr.k[tile][g * (D / 64) + cc], s.q[0][cc], a);
+    } else {
+      const u32x4 w = kr.k[tile][g];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 k = {E::template from_fp8x2<false>(w[2 * h]), E::template from_fp8x2<true>(w[2 * h]),
+                         E::template from_fp8x2<false>(w[2 * h + 1]), E::template from_fp8x2<true>(w[2 * h + 1])};
+        a = E::mfma(k, s.q[0][h], a);
+      }
+    }
+    x[g] = a;
+  }
+  f32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[0][e]), __float_as_uint(x[1][e]), false, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)r[1], 0x128, 0xf, 0xf, false);  // row_ror:8
+    o[e] = __uint_as_float(r[0]) + __int_as_float(hi);
+  }
+  return o;
+}
+
 // Scores of one chunk and the online-softmax update; returns the P^T B operands.
 // MASKED = false only when every token of the chunk is visible to every valid row.
 // LAZY: skip the accumulator rescale when no row max moved (a uniform branch; exact, and a
 // win for decode where the max settles early); otherwise the body is straight-line so the
 // row tiles' dependency chains interleave.
-template <class E, int D, int NT, bool MASKED, bool LAZY = true, class KR>
+template <class E, int D, int NT, bool MASKED, bool LINES, bool LAZY = true, class KR>
 __device__ __forceinline__ void chunk_scores(WaveState<D, NT>& s, const KR& kr, const PAParams& p,
                                              const ChunkRef& c, u32x4 pt[NT]) {
   const int j = (threadIdx.x & 63) >> 4;
   f32x4 st[NT][2];
-  if constexpr (std::is_same_v<KR, KRegs<D>>) {
+  if constexpr (LINES) {
+#pragma unroll
+    for (int tile = 0; tile < 2; ++tile) st[0][tile] = line_scores<E, D>(s, kr, tile);
+  } else if constexpr (std::is_same_v<KR, KRegs<D>>) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -533,18 +628,18 @@ __device__ __forceinline__ void chunk_pv(WaveState<D, NT>& s, VRegs8<D>& vr, con
 // The body is straight-line (masks always applied, loads unconditional) and the loads are
 // pinned in the order K(c+1), V(c+1) with scheduling barriers, so each s_waitcnt waits for
 // exactly the operand it guards while the other half of the next chunk stays in flight.
-template <class E, int D, int NT, bool KV8 = false, bool NTL = true>
+template <class E, int D, int NT, bool KV8 = false, bool NTL = true, bool LINES = false>
 __device__ __forceinline__ void run_chunks(WaveState<D, NT>& s, const PAParams& p, const int64_t* btrow, int kvh,
                                            int tok_begin, int stride, int tok_hi, int data_end) {
   if (tok_begin >= tok_hi) return;
   const int page_end = (tok_hi + p.BS - 1) / p.BS;
-  const LaneOffsets lo = lane_offsets<D, KV8>(p);
+  const LaneOffsets lo = lane_offsets<D, KV8, LINES>(p);
   PageWindow pw;
   load_window(pw, p, btrow, tok_begin / p.BS, page_end);
   ChunkRef c = chunk_ref(pw, p, btrow, tok_begin, tok_hi, page_end);
   std::conditional_t<KV8, KRegs8<D>, KRegs<D>> kr;
   std::conditional_t<KV8, VRegs8<D>, VRegs<D>> vr;
-  load_k<D, NTL>(kr, p, c, kvh, lo.k);
+  load_k<D, NTL, LINES>(kr, p, c, kvh, lo.k);
   __builtin_amdgcn_sched_barrier(0);
   load_v<D, NTL>(vr, p, c, kvh, lo.v);
   __builtin_amdgcn_sched_barrier(0);
@@ -553,9 +648,9 @@ __device__ __forceinline__ void run_chunks(WaveState<D, NT>& s, const PAParams& 
   while (c.tok0 + stride < tok_hi) {
     const ChunkRef cn = chunk_ref(pw, p, btrow, c.tok0 + stride, tok_hi, page_end);
     u32x4 pt[NT];
-    chunk_scores<E, D, NT, true>(s, kr, p, c, pt);
+    chunk_scores<E, D, NT, true, LINES>(s, kr, p, c, pt);
     __builtin_amdgcn_sched_barrier(0);
-    load_k<D, NTL>(kr, p, cn, kvh, lo.k);
+    load_k<D, NTL, LINES>(kr, p, cn, kvh, lo.k);
     __builtin_amdgcn_sched_barrier(0);
     chunk_pv<E, D, NT, true>(s, vr, c, data_end, pt);
     __builtin_amdgcn_sched_barrier(0);
@@ -564,7 +659,7 @@ __device__ __forceinline__ void run_chunks(WaveState<D, NT>& s, const PAParams& 
     c = cn;
   }
   u32x4 pt[NT];
-  chunk_scores<E, D, NT, true>(s, kr, p, c, pt);
+  chunk_scores<E, D, NT, true, LINES>(s, kr, p, c, pt);
   chunk_pv<E, D, NT, true>(s, vr, c, data_end, pt);
 }
 
@@ -1134,9 +1229,19 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
     const int tok_lo = skip + (int)(pos - seg_beg) * kChunk;
     const int tok_hi = min(skip + (int)(y - seg_beg) * kChunk, sv.kv_total);
     WaveState<D, NT> st;
-    load_q<D, NT, KV8>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
     const int64_t* btrow = p.bt + (int64_t)seq * p.bt_rs;
-    run_chunks<E, D, NT, KV8>(st, p, btrow, kvh, tok_lo, kChunk, tok_hi, sv.kv_total);
+    bool lines = false;
+    if constexpr (NT == 1 && NX == 1 && can_read_lines<D, KV8>()) {
+      lines = R <= kLineRows && (KV8 || b - a <= kLineUnitChunks);
+      if (lines) {
+        load_q<D, NT, KV8, true>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
+        run_chunks<E, D, NT, KV8, true, true>(st, p, btrow, kvh, tok_lo, kChunk, tok_hi, sv.kv_total);
+      }
+    }
+    if (!lines) {
+      load_q<D, NT, KV8>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
+      run_chunks<E, D, NT, KV8>(st, p, btrow, kvh, tok_lo, kChunk, tok_hi, sv.kv_total);
+    }
     const bool whole = pos == seg_beg && y == seg_end && !member;
     const int64_t slot = (int64_t)seq * NHG + hg + unit;
     write_rows<E, D, NT, (KV8 && NT > 1)>(st, p, sv, R, 0, kvh, !whole, p.ws_acc, p.ws_ml, (slot * p.HGW + hw) * p.RS,
@@ -1179,7 +1284,8 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
 // lane-partial sums; wave 0 then writes the normalised rows. Nothing goes through the
 // workspace and no merge launch follows: a batch this small is bound by latency, and the
 // merge launch was a third of it.
-template <class E, int D, bool KV8>
+// LINES: whole-line, non-temporal K/V loads for up to 8 rows (short_lines below).
+template <class E, int D, bool KV8, bool LINES>
 __global__ __launch_bounds__(256) void pa_decode_short_kernel(PAParams p) {
   constexpr int NI = D / 16;
   __shared__ f32x4 x_acc[kWavesPerWG - 1][NI][64];
@@ -1191,9 +1297,14 @@ __global__ __launch_bounds__(256) void pa_decode_short_kernel(PAParams p) {
   if (sv.q_len == 0 || sv.q_len > p.QS) return;  // uniform over the workgroup
   const int R = sv.q_len * p.G;
   WaveState<D, 1> st;
-  load_q<D, 1, KV8>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
   const int64_t* btrow = p.bt + (int64_t)seq * p.bt_rs;
-  run_chunks<E, D, 1, KV8, false>(st, p, btrow, kvh, w * kChunk, kWavesPerWG * kChunk, sv.kv_total, sv.kv_total);
+  if (LINES && R <= kLineRows) {
+    load_q<D, 1, KV8, LINES>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
+    run_chunks<E, D, 1, KV8, true, LINES>(st, p, btrow, kvh, w * kChunk, kWavesPerWG * kChunk, sv.kv_total, sv.kv_total);
+  } else {
+    load_q<D, 1, KV8>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
+    run_chunks<E, D, 1, KV8, false>(st, p, btrow, kvh, w * kChunk, kWavesPerWG * kChunk, sv.kv_total, sv.kv_total);
+  }
   if (w > 0) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) x_acc[w - 1][i][lane] = st.acc[0][i];
@@ -2522,7 +2633,11 @@ template <class E, int D, bool KV8>
 static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipStream_t s, LaunchLog& log) {
   int err = 0;
   if (plan.short_decode) {
-    hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8>), dim3(p.Hkv, p.B), dim3(256), 0, s, p);
+    if (can_read_lines<D, KV8>() && (int64_t)p.B * p.Hkv * D >= kShortLines)
+      hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, can_read_lines<D, KV8>()>), dim3(p.Hkv, p.B), dim3(256), 0, s,
+                         p);
+    else
+      hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, false>), dim3(p.Hkv, p.B), dim3(256), 0, s, p);
     if ((err = (int)hipGetLastError())) return err;
     log.after_launch(1, s);
     return 0;

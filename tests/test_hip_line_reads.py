@@ -1,0 +1,58 @@
+"""Decode through whole-line K reads (up to 8 query rows per kv head) and past them: the short
+decode of batches large enough to take them, with stale slots that hold NaN, at row counts on
+both sides of 8, over 16-bit and E4M3 caches; and the stream-K decode on both sides of the unit
+length up to which 16-bit caches take them."""
+
+from __future__ import annotations
+
+import random
+
+import pytest
+import torch
+
+from kvserve_amd import HipAttention, last_launch_kernels, workloads
+from oracle import fp8, torch_reference
+from tests import paged_check as pc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(("heads", "q"), [((32, 8), 1), ((32, 8), 2), ((32, 8), 3), ((16, 16), 8), ((64, 8), 1)])
+def test_short_decode(hip_device, heads, q, head_dim, e4m3):
+    rng = random.Random(q)
+    B = 40  # B Hkv D >= 16384 at every shape
+    ctx = [0, 1, 7, 8, 15, 16, 17, 31, 32, 33, 40, 1024 - q] + [rng.randint(0, 700) for _ in range(B - 12)]
+    w = workloads.custom("lines", [q] * B, ctx, *heads, head_dim, 16, seed=q)
+    b = workloads.materialize(w, torch.bfloat16, hip_device, seed=q)
+    for t, n in zip(w.tables, w.seq_lens):  # slots past a sequence's keys hold anything
+        if n % 16:
+            b.k_cache[t[n // 16], n % 16 :] = float("nan")
+            b.v_cache[t[n // 16], n % 16 :] = float("nan")
+    if e4m3:
+        k, v = fp8.quantize(b.k_cache, 1.0).to(hip_device), fp8.quantize(b.v_cache, 0.5).to(hip_device)
+        HipAttention.write_kv(k, v, b.k_new, b.v_new, b.meta.slot_mapping, k_scale=1.0, v_scale=0.5)
+        out = HipAttention.forward(b.q, k, v, b.meta, w.scale, k_scale=1.0, v_scale=0.5)
+        kf, vf = fp8.dequantize(k.cpu(), 1.0), fp8.dequantize(v.cpu(), 0.5)
+    else:
+        out = pc.attend(b)
+        kf, vf = b.k_cache.float().cpu(), b.v_cache.float().cpu()
+    assert last_launch_kernels() == ["decode"]
+    m = b.meta
+    ref = torch_reference.forward(b.q.float().cpu(), kf.nan_to_num(), vf.nan_to_num(), m.block_tables.cpu(),
+                                  m.seq_lens.cpu(), m.query_lens.cpu(), w.scale)  # fmt: skip
+    assert (out.float().cpu() - ref).abs().max().item() <= pc.TOL_16BIT
+
+
+@pytest.mark.parametrize("ctx", [4000, 4200, 12000])
+@pytest.mark.parametrize(("heads", "q"), [((32, 8), 1), ((32, 8), 3), ((8, 1), 1)])
+def test_stream_k_decode(hip_device, heads, q, ctx):
+    # 128 units of 8-head groups: 32 sequences of 4096 keys give 32 chunks a unit
+    B = 32 if heads[1] == 8 else 8
+    lens = [ctx + 37 * i for i in range(B)] if ctx < 5000 else [ctx] + [200 + 61 * i for i in range(B - 1)]
+    w = workloads.custom("stream", [q] * B, lens, *heads, 128, 16, seed=7)
+    b = workloads.materialize(w, torch.bfloat16, hip_device, seed=7)
+    out = pc.attend(b)
+    assert "reduce" in last_launch_kernels()
+    assert pc.max_err_vs_oracle(b, out, [0, 1, B // 2, B - 1]) <= pc.TOL_16BIT
