@@ -131,6 +131,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
 
 _lib: ctypes.CDLL | None = None
 _fast = None
+_calls = None
 _lock = threading.Lock()
 
 
@@ -169,6 +170,19 @@ def load() -> ctypes.CDLL:
             raise RuntimeError(
                 f"kvserve_amd/_kvhfast is not built ({e}): build it with `python -m kvserve_amd.build`."
             ) from e
+        global _calls
+        import torch  # the libraries _kvhtorch links to
+
+        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw_stream is not None:
+            try:
+                from kvserve_amd import _kvhtorch
+            except ImportError as e:
+                raise RuntimeError(
+                    f"kvserve_amd/_kvhtorch is not built ({e}): build it with `python -m kvserve_amd.build`."
+                ) from e
+            _kvhtorch.bind(lib._handle, raw_stream)
+            _calls = _kvhtorch
         _kvhfast.bind(lib._handle)
         _fast = _kvhfast
         _lib = lib
@@ -180,6 +194,14 @@ def fast():
     if _fast is None:
         load()
     return _fast
+
+
+def calls():
+    """The per-step calls on tensors (_kvhtorch), bound to the loaded library; None when this PyTorch
+    does not hand out stream handles (a build without a GPU backend)."""
+    if _lib is None:
+        load()
+    return _calls
 
 
 def strerror(status: int) -> str:

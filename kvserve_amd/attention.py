@@ -130,6 +130,12 @@ def _check_index(t: torch.Tensor, name: str, dim: int) -> None:
     _require(t.dim() == dim and t.stride(-1) == 1, f"{name} must be {dim}-d with a contiguous last dim")
 
 
+def _calls():
+    """The calls on tensors in C++ (_lib.calls): each returns None for whatever is not a plain, valid
+    call, and the method below then does it step by step, with its own errors."""
+    return _lib._calls if _lib._lib is not None else None
+
+
 class HipAttention:
     """Paged attention on hand-written gfx950 kernels (decode split-K + reduce, MFMA prefill).
 
@@ -161,6 +167,13 @@ class HipAttention:
         Slots outside the pool are skipped instead of raising. float8_e4m3fn caches store
         (x / scale).clamp(-448, 448).to(float8_e4m3fn) with the given scales, bit for bit.
         """
+        calls = _calls()
+        if calls is not None:
+            r = calls.write_kv(k_cache, v_cache, k, v, slots, k_scale, v_scale)
+            if r is True:
+                return
+            if r is not None:
+                _lib.check(r, "kvh_reshape_and_cache_fp8" if k_cache.dtype == FP8 else "kvh_reshape_and_cache")
         num_blocks, block_size, num_kv_heads, head_dim, kcs, vcs, dev = _cache_layout(k_cache, v_cache)
         fp8 = _kv_format(k_cache, v_cache, k_scale, v_scale)
         _on_device(dev, k=k, v=v, slot_mapping=slots)
@@ -215,6 +228,13 @@ class HipAttention:
         RoPE(q) as [T, num_heads, head_dim] (in `out` if given), bit-identical to the
         reference's bf16/fp16/fp32 torch operations.
         """
+        calls = _calls()
+        if calls is not None:
+            r = calls.rope_and_cache(qkv, positions, cos, sin, k_cache, v_cache, slots, num_heads, out, k_scale, v_scale)
+            if type(r) is int:
+                _lib.check(r, "kvh_rope_and_cache_fp8" if k_cache.dtype == FP8 else "kvh_rope_and_cache")
+            if r is not None:
+                return r
         num_blocks, block_size, num_kv_heads, head_dim, kcs, vcs, dev = _cache_layout(k_cache, v_cache)
         fp8 = _kv_format(k_cache, v_cache, k_scale, v_scale)
         _on_device(dev, qkv=qkv, positions=positions, cos=cos, sin=sin, slot_mapping=slots)
@@ -309,6 +329,14 @@ class HipAttention:
     ) -> torch.Tensor:
         """q: [T, H, D]; caches: [num_blocks, block_size, H_kv, D]. Returns [T, H, D] (in `out` if given).
         float8_e4m3fn caches hold keys / values as e4m3 * k_scale / v_scale (q and out bf16 or fp16)."""
+        calls = _calls()
+        if calls is not None:
+            r = calls.forward(q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.query_start_loc,
+                              meta.max_query_len, scale, out, k_scale, v_scale)  # fmt: skip
+            if type(r) is int:
+                _lib.check(r, "kvh_paged_attention_fp8" if k_cache.dtype == FP8 else "kvh_paged_attention")
+            if r is not None:
+                return r
         num_blocks, block_size, num_kv_heads, head_dim, kcs, vcs, dev = _cache_layout(k_cache, v_cache)
         fp8 = _kv_format(k_cache, v_cache, k_scale, v_scale)
         tables, seq_lens, qsl = meta.block_tables, meta.seq_lens, meta.query_start_loc

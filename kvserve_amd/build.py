@@ -106,6 +106,32 @@ def build_fastcall(verbose: bool = False) -> Path:
     return out
 
 
+def build_torch_calls(verbose: bool = False) -> Path:
+    """The per-step calls on tensors (csrc/pytorch_calls.cpp -> _kvhtorch*.so next to this file),
+    compiled with the host compiler against the installed PyTorch's C++ headers; PyTorch's
+    libraries are those the process has loaded, libkvhip's symbols are resolved at run time."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    out = PKG / ("_kvhtorch" + sysconfig.get_config_var("EXT_SUFFIX"))
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler for the _kvhtorch binding")
+    tmp = out.with_suffix(".so.tmp")
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", *[f"-isystem{d}" for d in include_paths()],
+           str(CSRC / "pytorch_calls.cpp"), *[f"-L{d}" for d in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10",
+           "-ldl", "-o", str(tmp)]  # fmt: skip
+    if verbose:
+        print(" ".join(cmd))
+    _run(cmd)
+    os.replace(tmp, out)
+    return out
+
+
 def build(
     verbose: bool = False, extra_flags: list[str] | None = None, out: Path | None = None, build_dir: Path | None = None
 ) -> Path:
@@ -156,6 +182,7 @@ def build(
     os.replace(tmp, lib)  # atomic: a process that already mapped the old file keeps it
     if out is None:
         build_fastcall(verbose)
+        build_torch_calls(verbose)
     return lib
 
 
