@@ -155,14 +155,19 @@ constexpr bool can_read_lines() {
 }
 constexpr int kLineRows = 8;
 // Where whole-line reads pay (bf16, times in us without / with):
-//  * the stream-K decode over E4M3 caches: 64 sequences of 1023-8191 keys, step 114.9 / 113.6; over
-//    16-bit caches only in units of up to kLineUnitChunks chunks: 16 sequences of 200-2200 keys 29.7 /
-//    28.5, but the 64 sequences (73 chunks a unit) 200.7 / 201.7, 512 sequences 801 / 811;
-//  * the short decode, together with non-temporal loads, from kShortLines = B Hkv D: 128 x 1000 keys
-//    102 / 88 (D = 128), 60 / 52 (D = 64), 32 x 1000 28.2 / 24.9, 16 x 500 12.4 / 11.3; below it the
-//    caches' half-line hits win (8 x 500 keys, D = 64: 7.3 / 8.5).
-constexpr int kLineUnitChunks = 32;
-constexpr int64_t kShortLines = 16384;
+//  * the stream-K decode over E4M3 caches in units of more than kLineMinChunks8 chunks: 64 sequences of
+//    4000-8000 keys 141.4 / 139.4, 19 of 3000-6000 (10 chunks a unit) 44.2 / 43.6, but over 4 kv
+//    heads (5 a unit) 36.7 / 37.5, and 4 sequences of 2000-4000 keys over 16 (3 a unit) 25.7 / 26.2;
+//    over 16-bit caches in units of up to kLineUnitChunks: 16 sequences of 200-2200 keys 29.7 / 28.5,
+//    but 64 of 1023-8191 (73 a unit) 200.7 / 201.7, 512 sequences 801 / 811;
+//  * the short decode, together with non-temporal loads, over 16-bit caches from kShortLines = B Hkv D:
+//    128 x 1000 keys 102 / 88 (D = 128), 60 / 52 (D = 64), 32 x 1000 28.2 / 24.9, 16 x 500
+//    12.4 / 11.3; below it the caches' half-line hits win (8 x 500 keys, D = 64: 7.3 / 8.5). Over E4M3
+//    caches from kShortLines8 elements of the tables' K (B Hkv D W BS): 128 x 1000 keys 57.1 / 49.6 (8
+//    kv heads), 29.5 / 27.1 (4), 131 x 300 39.1 / 34.0 (16), but 131 x 300 20.7 / 21.5 and 32 x 1000
+//    16.3 / 17.8 (8).
+constexpr int kLineUnitChunks = 32, kLineMinChunks8 = 8;
+constexpr int64_t kShortLines = 16384, kShortLines8 = 48 << 20;
 
 template <int D, bool KV8 = false, bool LINES = false>
 __device__ __forceinline__ LaneOffsets lane_offsets(const PAParams& p) {
@@ -1232,7 +1237,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
     const int64_t* btrow = p.bt + (int64_t)seq * p.bt_rs;
     bool lines = false;
     if constexpr (NT == 1 && NX == 1 && can_read_lines<D, KV8>()) {
-      lines = R <= kLineRows && (KV8 || b - a <= kLineUnitChunks);
+      lines = R <= kLineRows && (KV8 ? b - a > kLineMinChunks8 : b - a <= kLineUnitChunks);
       if (lines) {
         load_q<D, NT, KV8, true>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
         run_chunks<E, D, NT, KV8, true, true>(st, p, btrow, kvh, tok_lo, kChunk, tok_hi, sv.kv_total);
@@ -2633,7 +2638,8 @@ template <class E, int D, bool KV8>
 static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipStream_t s, LaunchLog& log) {
   int err = 0;
   if (plan.short_decode) {
-    if (can_read_lines<D, KV8>() && (int64_t)p.B * p.Hkv * D >= kShortLines)
+    const int64_t rows = (int64_t)p.B * p.Hkv * D;
+    if (can_read_lines<D, KV8>() && (KV8 ? rows * p.W * p.BS >= kShortLines8 : rows >= kShortLines))
       hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, can_read_lines<D, KV8>()>), dim3(p.Hkv, p.B), dim3(256), 0, s,
                          p);
     else

@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize(("heads", "q"), [((32, 8), 1), ((32, 8), 2), ((32, 8), 3), ((16, 16), 8), ((64, 8), 1)])
 def test_short_decode(hip_device, heads, q, head_dim, e4m3):
     rng = random.Random(q)
-    B = 40  # B Hkv D >= 16384 at every shape
+    B = 64 if e4m3 else 40  # B Hkv D >= 16384; over E4M3 caches, D = 128, B Hkv D 1024 >= 48 Mi
     ctx = [0, 1, 7, 8, 15, 16, 17, 31, 32, 33, 40, 1024 - q] + [rng.randint(0, 700) for _ in range(B - 12)]
     w = workloads.custom("lines", [q] * B, ctx, *heads, head_dim, 16, seed=q)
     b = workloads.materialize(w, torch.bfloat16, hip_device, seed=q)
