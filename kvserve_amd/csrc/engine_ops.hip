@@ -302,17 +302,18 @@ template <class E, SkinnyForm F, int MT, bool GLU>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_rs,
                                                                         const uint16_t* __restrict__ w, int64_t w_rs,
                                                                         uint16_t* __restrict__ y, int64_t y_rs, int m,
-                                                                        int k, int n, int ks, int vec) {
+                                                                        int k, int n, int slices, int vec) {
   constexpr int THREADS = 64 * kSkinnyWaves;
   constexpr int TR = skinny_rows(F), COLS = GLU ? TR / 2 : TR;  // weight rows and outputs of a tile
   extern __shared__ __attribute__((aligned(16))) char lds[];
   f32x4(*red)[MT][64] = (f32x4(*)[MT][64])lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = skinny_row<F>(lane);
-  const int tiles = kSkinnyWaves / ks;  // of this workgroup
+  const int ks = F == kSkinnyShared ? slices : kSkinnyWaves, lks = __builtin_ctz(ks);  // a power of two
+  const int tiles = kSkinnyWaves >> lks;  // of this workgroup
   const int64_t tile0 = (int64_t)blockIdx.x * tiles, all = n / COLS;
-  const int64_t n0 = min(tile0 + wave / ks, all - 1) * COLS;  // waves past the last tile repeat it
-  const int slice = wave % ks, len = k / ks;
+  const int64_t n0 = min(tile0 + (wave >> lks), all - 1) * COLS;  // waves past the last tile repeat it
+  const int slice = wave & (ks - 1), len = k >> lks;
   const int64_t wrow = GLU ? (i < COLS ? n0 + i : n + n0 + i - COLS) : n0 + i;
   const uint16_t* wr = w + wrow * w_rs + slice * len + skinny_k<F>(lane);
   f32x4 acc[MT];
@@ -351,13 +352,13 @@ int launch_skinny_t(const void* x, int64_t x_rs, const void* w, int64_t w_rs, vo
                     int k, hipStream_t s) {
   const int64_t rows = GLU ? 2 * (int64_t)n : n;
   const int ks = skinny_slices(rows, k, m), per = kSkinnyWaves / ks;
-  const int tiles = (int)(rows / skinny_rows(skinny_form(rows, m)));
+  const int tiles = (int)(rows / skinny_rows(skinny_form(rows, k, m)));
   const dim3 grid((unsigned)((tiles + per - 1) / per)), block(64 * kSkinnyWaves);
   const int vec = (((uintptr_t)y | (uintptr_t)(2 * y_rs)) & 7) == 0;  // 8-byte stores
 #define KVH_LAUNCH_SKINNY(F, MT)                                                                                    \
   hipLaunchKernelGGL((skinny_gemm_kernel<E, F, MT, GLU>), grid, block, (skinny_lds_bytes<F, MT>(ks)), s,             \
                      (const uint16_t*)x, x_rs, (const uint16_t*)w, w_rs, (uint16_t*)y, y_rs, m, k, n, ks, vec)
-  switch (skinny_form(rows, m)) {
+  switch (skinny_form(rows, k, m)) {
     case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
     case kSkinnyFull:
       switch ((m + 15) / 16) {

@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void gemv_rope_cache_kernel(GemvRopeArgs a) {
 // i < NP, h D + d0 + D / 2 + i - NP for i >= NP, and MT B tiles of x; the partial tiles meet in LDS,
 // are summed in slice order and go through rope_pair_out.
 template <int DT, SkinnyForm F, int MT, bool KV8>
-__global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(GemvRopeArgs a, int m, int ks) {
+__global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(GemvRopeArgs a, int m, int slices) {
   using E = std::conditional_t<DT == 2, BF16, F16>;
   constexpr int THREADS = 64 * kSkinnyWaves, TR = skinny_rows(F), NP = TR / 2;
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -324,12 +324,13 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(Ge
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = skinny_row<F>(lane);
   const int half = a.D / 2;
-  const int tiles = kSkinnyWaves / ks;  // of this workgroup
+  const int ks = F == kSkinnyShared ? slices : kSkinnyWaves, lks = __builtin_ctz(ks);  // a power of two
+  const int tiles = kSkinnyWaves >> lks;  // of this workgroup
   const int tile0 = blockIdx.x * tiles, all = (a.H + 2 * a.Hkv) * half / NP;
-  const int p0 = min(tile0 + wave / ks, all - 1) * NP;  // first pair; waves past the last tile repeat it
+  const int p0 = min(tile0 + (wave >> lks), all - 1) * NP;  // first pair; waves past the last tile repeat it
   const int h = p0 / half, d0 = p0 % half;
   const int64_t wrow = (int64_t)h * a.D + d0 + (i < NP ? i : half + i - NP);
-  const int slice = wave % ks, len = a.k / ks;
+  const int slice = wave & (ks - 1), len = a.k >> lks;
   const uint16_t* wr = a.w + wrow * a.w_rs + slice * len + skinny_k<F>(lane);
   f32x4 acc[MT];
 #pragma unroll
@@ -358,11 +359,11 @@ static int launch_gemv_rope_dt(const GemvRopeArgs& a, int m, hipStream_t s) {
   if (m > 4) {  // the skinny form
     const int64_t rows = 2 * (int64_t)waves;
     const int ks = skinny_slices(rows, a.k, m), per = kSkinnyWaves / ks;
-    const int tiles = (int)(rows / skinny_rows(skinny_form(rows, m)));
+    const int tiles = (int)(rows / skinny_rows(skinny_form(rows, a.k, m)));
     const dim3 g2((unsigned)((tiles + per - 1) / per)), b2(64 * kSkinnyWaves);
 #define KVH_LAUNCH_SKINNY(F, MT) \
   hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, F, MT, KV8>), g2, b2, (skinny_lds_bytes<F, MT>(ks)), s, a, m, ks)
-    switch (skinny_form(rows, m)) {
+    switch (skinny_form(rows, a.k, m)) {
       case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
       case kSkinnyFull:
         switch ((m + 15) / 16) {

@@ -3,53 +3,26 @@
 // keep HBM busy over the range of shapes (times on (n, k), cold weights, bf16):
 //
 //  kSkinnyFull    16 weight rows as the A operand, a load reading 64 bytes of each, 16 rows of x
-//                 per B tile straight from the caches; k split over 8 waves. 9 to 64 rows of x
-//                 against weights of few rows.
+//                 per B tile straight from the caches; k split over 8 waves. Weights of few rows.
 //  kSkinnyHalf    m <= 8: the A operand is 8 weight rows twice, rows i and i + 8 the same row at
 //                 two neighbouring 8-element chunks, and the B operand 8 rows of x likewise: the
 //                 products of equal halves sum to the result, those of unequal ones are dropped.
 //                 A load then reads whole 128-byte lines of 8 rows, non-temporally (nothing reads
 //                 the weight again in this step), and twice the tiles fill the chip: (2048, 8192)
-//                 at 8 rows 16.0 -> 11.0 us, (2048, 2048) 5.7 -> 4.8.
+//                 at 8 rows 14.6 -> 10.4 us, (2048, 2048) 5.7 -> 4.9.
 //  kSkinnyShared  the half tiles for any m, ceil(m / 8) B tiles, with x staged in LDS in chunks,
 //                 one chunk ahead, and shared by the workgroup's tiles. Read from the caches by
 //                 every wave, x took the L1's bandwidth from the weight: (128256, 4096) 240 us at
-//                 8 rows and 399 at 32, against 185 and 219 with x left out. For weights of
-//                 kSkinnySharedRows rows or more, whose tiles fill the chip with k split little.
+//                 8 rows and 399 at 32, against 185 and 219 with x left out. For weights of many
+//                 rows, whose tiles fill the chip with k split little.
 #pragma once
 
 #include <type_traits>
 
 #include "kvh_device.h"
+#include "skinny_form.h"
 
 namespace kvh {
-
-constexpr int kSkinnyWaves = 8;       // waves of a workgroup: `ks` for each of its tiles
-enum SkinnyForm { kSkinnyFull, kSkinnyHalf, kSkinnyShared };
-constexpr int64_t kSkinnySharedRows = 8192;
-
-inline SkinnyForm skinny_form(int64_t rows, int m) {
-  return rows >= kSkinnySharedRows ? kSkinnyShared : (m <= 8 ? kSkinnyHalf : kSkinnyFull);
-}
-// weight rows (and x rows of a B tile) of a tile, k per MFMA step and per batch of 4 steps, k of a
-// staged chunk of x
-constexpr int skinny_rows(SkinnyForm f) { return f == kSkinnyFull ? 16 : 8; }
-constexpr int skinny_step(SkinnyForm f) { return f == kSkinnyFull ? 32 : 64; }
-constexpr int skinny_batch(SkinnyForm f) { return 4 * skinny_step(f); }
-constexpr int kSkinnyChunk = 512;
-
-// k-slices per tile of a weight of `rows` rows: the smallest power of two that gives the
-// chip 8 waves per CU (16 of half tiles), at most kSkinnyWaves (with x shared 2, or 1 above 32 rows: its LDS), slices
-// being whole batches or chunks. A function of the weight's shape and of m alone, so that a projection and its fused
-// forms sum in one order.
-inline int skinny_slices(int64_t rows, int64_t k, int m) {
-  const SkinnyForm f = skinny_form(rows, m);
-  const int most = f == kSkinnyShared ? (m <= 32 ? 2 : 1) : kSkinnyWaves, unit = f == kSkinnyShared ? kSkinnyChunk : skinny_batch(f);
-  const int target = f == kSkinnyHalf ? 4096 : 2048;  // (6144, 4096) at 8 rows: half tiles 17.9 us at 2048, 14.7 at 4096
-  int ks = 1;
-  while (ks < most && rows / skinny_rows(f) * ks < target && k % (2 * ks * unit) == 0) ks *= 2;
-  return ks;
-}
 
 // LDS of a workgroup: x's chunks of all slices twice (each row padded so that the rows of an
 // operand read fall on different banks), or the partial tiles at the end.
@@ -190,7 +163,9 @@ template <SkinnyForm F, int MT>
 __device__ __forceinline__ f32x4 skinny_sum(const f32x4 (*red)[MT][64], int ks, int t, int l) {
   f32x4 o = red[0][t][l];
   if constexpr (F != kSkinnyFull) o += red[0][t][l + 40];
-  for (int v = 1; v < ks; ++v) {
+#pragma unroll
+  for (int v = 1; v < (F == kSkinnyShared ? 2 : kSkinnyWaves); ++v) {
+    if (v >= ks) break;
     o += red[v][t][l];
     if constexpr (F != kSkinnyFull) o += red[v][t][l + 40];
   }
