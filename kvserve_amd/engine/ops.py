@@ -61,20 +61,25 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 def skinny_wins(m: int, n: int, k: int) -> bool:
     """Where kvh_gemm_skinny beats hipBLASLt, by weight shape (n, k), cold weights on MI355X, bf16
     (skinny / hipBLASLt in us):
-      up to 8 rows    weights of 8192 rows or more ((28672, 4096) 44 / 62, (128256, 2048) 96 / 117,
-                      (128256, 4096) 178 / 191, (16384, 2048) 16 / 18.8) and up to 40 MB ((2048,
-                      8192) 10 / 12.7, (4096, 4096) 10 / 15.5); not (4096, 14336) 28 / 26
-      up to 16 rows   the large ones (44 / 60, 101 / 128, 175 / 194, 16 / 17.4), up to 13 MB
-                      ((3072, 2048) 6.6 / 11.5) and 4096 rows up to 40 MB ((4096, 4096) 11 / 15.6);
-                      not (2048, 8192) 17 / 13.3
-      up to 32 rows   up to 13 MB ((3072, 2048) 8.5 / 11.7); not (128256, 4096) 212 / 203"""
+      up to 8 rows    weights of 8192 rows or more ((28672, 4096) 44 / 66, (128256, 2048) 95 / 101,
+                      (128256, 4096) 178 / 191, (16384, 2048) 15 / 18) and up to 80 MB: at 8 rows (2048,
+                      8192) 10.2 / 12.9, (4096, 4096) 9.4 / 15.7, (4096, 5120) 10.8 / 19.3, (6144, 4096)
+                      13.3 / 14.8, (7168, 4096) 14.0 / 15.5, (4096, 8192) 15.7 / 16.1, (7168, 5120)
+                      16.3 / 17.0; level or up to 5% behind at (5120, 5120) 15.1 / 14.9, (3072, 8192)
+                      14.8 / 14.1, (2560, 9216) 16.1 / 15.4; not (3584, 11264) 19.8 / 19.0
+      up to 16 rows   the large ones (45 / 64, 99 / 99, 175 / 194, 16 / 18; behind at (9216, 8192) 37 /
+                      34), up to 13 MB ((3072, 2048) 6.4 / 11.4), 4096 rows of k up to 4096, whose tiles
+                      fit the CUs once ((4096, 4096) 10.4 / 15.7, (3072, 4096) 10.1 / 15.2), and 4096
+                      rows or more up to 30 MB ((7168, 2048) 10.4 / 12.8); not (6144, 3072) 13.7 / 12.0,
+                      (5120, 4096) 17.4 / 14.1 or (2048, 8192) 17 / 13.3
+      up to 32 rows   up to 13 MB ((3072, 2048) 8.1 / 11.6); not (128256, 4096) 212 / 203"""
     if n % 16 or k % 1024:
         return False
     w_bytes = 2 * n * k
     if m <= 8:
-        return n >= 8192 or w_bytes <= 40e6
+        return n >= 8192 or w_bytes <= 80e6
     if m <= 16:
-        return n >= 8192 or w_bytes <= 13e6 or (n >= 4096 and w_bytes <= 40e6)
+        return n >= 8192 or w_bytes <= 13e6 or (n <= 4096 and k <= 4096) or (n >= 4096 and w_bytes <= 30e6)
     return m <= 32 and w_bytes <= 13e6
 
 

@@ -1,6 +1,6 @@
 """Which form of the skinny GEMM a weight takes (csrc/skinny_form.h), compiled for the host: the shapes
 where one form was measured against another take the faster one, and every choice is one the kernels can
-run (whole batches or chunks of k per slice)."""
+run (whole batches or chunks of k per slice). And where the engine takes the kernel rather than hipBLASLt."""
 
 from __future__ import annotations
 
@@ -10,6 +10,8 @@ import subprocess
 from pathlib import Path
 
 import pytest
+
+from kvserve_amd.engine.ops import skinny_wins
 
 CSRC = Path(__file__).resolve().parent.parent / "kvserve_amd/csrc"
 FULL, HALF, SHARED = 0, 1, 2
@@ -69,3 +71,18 @@ def test_every_choice_can_run(lib):
                 assert ks == lib.waves() if f != SHARED else ks in ((1, 2) if m <= 32 else (1,))
                 assert k % (ks * (lib.chunk() if f == SHARED else lib.batch(f))) == 0
                 assert m <= 8 or f != HALF
+
+
+# rows of x, (n, k), whether the skinny kernel was faster than hipBLASLt (by 3% or more either way)
+ROUTED = [
+    (8, (4096, 5120), True), (8, (6144, 4096), True), (5, (7168, 4096), True), (8, (2048, 14336), True),
+    (8, (7168, 5120), True), (8, (28672, 4096), True), (8, (3584, 11264), False), (16, (4096, 4096), True),
+    (16, (3072, 4096), True), (16, (7168, 2048), True), (16, (5120, 3072), False), (16, (6144, 3072), False),
+    (16, (5120, 4096), False), (16, (2048, 8192), False), (16, (28672, 4096), True), (32, (3072, 2048), True),
+    (32, (4096, 8192), False), (33, (3072, 2048), False),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize(("m", "shape", "wins"), ROUTED)
+def test_the_engine_takes_the_faster_kernel(m, shape, wins):
+    assert skinny_wins(m, *shape) == wins
