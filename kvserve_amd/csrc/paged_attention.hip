@@ -38,6 +38,7 @@
 
 #include "kvh_device.h"
 #include "kvh_internal.h"
+#include "line_reads.h"
 #include "prefill_plan.h"
 
 namespace kvh {
@@ -147,28 +148,8 @@ struct LaneOffsets {
 // likewise (lane column n: row n % 8, chunk n / 8), which takes the columns that 8 rows or fewer
 // leave idle anyway: S is the sum of the products of equal halves (line_scores), in as many MFMAs
 // as before. A non-temporal load does not keep the line's other half for the next instruction, so
-// half-line reads ask the L2 twice for every line. Rows of 128 bytes or more: 16-bit caches, and
-// E4M3 caches at D = 128.
-template <int D, bool KV8>
-constexpr bool can_read_lines() {
-  return !KV8 || D == 128;
-}
-constexpr int kLineRows = 8;
-// Where whole-line reads pay (bf16, times in us without / with):
-//  * the stream-K decode over E4M3 caches in units of more than kLineMinChunks8 chunks: 64 sequences of
-//    4000-8000 keys 141.4 / 139.4, 19 of 3000-6000 (10 chunks a unit) 44.2 / 43.6, but over 4 kv
-//    heads (5 a unit) 36.7 / 37.5, and 4 sequences of 2000-4000 keys over 16 (3 a unit) 25.7 / 26.2;
-//    over 16-bit caches in units of up to kLineUnitChunks: 16 sequences of 200-2200 keys 29.7 / 28.5,
-//    but 64 of 1023-8191 (73 a unit) 200.7 / 201.7, 512 sequences 801 / 811;
-//  * the short decode, together with non-temporal loads, over 16-bit caches from kShortLines = B Hkv D:
-//    128 x 1000 keys 102 / 88 (D = 128), 60 / 52 (D = 64), 32 x 1000 28.2 / 24.9, 16 x 500
-//    12.4 / 11.3; below it the caches' half-line hits win (8 x 500 keys, D = 64: 7.3 / 8.5). Over E4M3
-//    caches from kShortLines8 elements of the tables' K (B Hkv D W BS): 128 x 1000 keys 57.1 / 49.6 (8
-//    kv heads), 29.5 / 27.1 (4), 131 x 300 39.1 / 34.0 (16), but 131 x 300 20.7 / 21.5 and 32 x 1000
-//    16.3 / 17.8 (8).
-constexpr int kLineUnitChunks = 32, kLineMinChunks8 = 8;
-constexpr int64_t kShortLines = 16384, kShortLines8 = 48 << 20;
-
+// half-line reads ask the L2 twice for every line. Rows of 128 bytes or more (can_read_lines); where they pay is
+// in line_reads.h.
 template <int D, bool KV8 = false, bool LINES = false>
 __device__ __forceinline__ LaneOffsets lane_offsets(const PAParams& p) {
   const int lane = threadIdx.x & 63;
@@ -1123,8 +1104,10 @@ __device__ __forceinline__ void write_job_x(int32_t* job, int pieces, int64_t sl
 // Decode class: NU * HGW / 4 workgroups of 4 waves; wave w of workgroup `block` is head w % HGW
 // of unit (4 block + w) / HGW. KV8: the cache is E4M3. NX: 16-row tiles of a cascade prefix
 // group (XR = 16 NX rows; 1 outside the cascade).
-template <class E, int D, int NT, bool KV8, int NX>
+// LINES: whole-line K reads where the launch's mean unit asks for them (line_units).
+template <class E, int D, int NT, bool KV8, int NX, bool LINES>
 __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
+  static_assert(!LINES || (NT == 1 && NX == 1));
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int gw = block * kWavesPerWG + wave;
@@ -1176,6 +1159,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
                         rounds ? kRound1Share : 1, rounds ? kRound2Share : 1);
   const int64_t a = split.begin(unit), b = split.begin(unit + 1);
   if (a >= b) return;
+  const bool lines = LINES && L == 0 && line_units(KV8, C, NUa);
 
   int64_t pos = a;
   if constexpr (NT == 1) {
@@ -1235,9 +1219,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
     const int tok_hi = min(skip + (int)(y - seg_beg) * kChunk, sv.kv_total);
     WaveState<D, NT> st;
     const int64_t* btrow = p.bt + (int64_t)seq * p.bt_rs;
-    bool lines = false;
-    if constexpr (NT == 1 && NX == 1 && can_read_lines<D, KV8>()) {
-      lines = R <= kLineRows && (KV8 ? b - a > kLineMinChunks8 : b - a <= kLineUnitChunks);
+    if constexpr (LINES) {
       if (lines) {
         load_q<D, NT, KV8, true>(st, p, sv.qs, R, 0, kvh, sv.ctx, sv.kv_total);
         run_chunks<E, D, NT, KV8, true, true>(st, p, btrow, kvh, tok_lo, kChunk, tok_hi, sv.kv_total);
@@ -1289,7 +1271,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
 // lane-partial sums; wave 0 then writes the normalised rows. Nothing goes through the
 // workspace and no merge launch follows: a batch this small is bound by latency, and the
 // merge launch was a third of it.
-// LINES: whole-line, non-temporal K/V loads for up to 8 rows (short_lines below).
+// LINES: whole-line, non-temporal K/V loads for up to 8 rows (launch_mfma_typed).
 template <class E, int D, bool KV8, bool LINES>
 __global__ __launch_bounds__(256) void pa_decode_short_kernel(PAParams p) {
   constexpr int NI = D / 16;
@@ -2350,7 +2332,7 @@ __device__ __forceinline__ bool prefill_start(const PAParams& p, int b, PreStart
 // / 4) + NUP): each writes where a prefill unit starts, under the decode work, and the prefill
 // launch behind it begins with one load. (Computed by the prefill workgroups themselves it was
 // on that launch's path: 512 decodes and four 384-token chunks over E4M3 caches 483 -> 492 us.)
-template <class E, int D, int NT, bool KV8, int NX>
+template <class E, int D, int NT, bool KV8, int NX, bool LINES>
 __global__ __launch_bounds__(256) void pa_decode_kernel(PAParams p) {
   const int b = blockIdx.x;
   if constexpr (NX == 1) {
@@ -2365,7 +2347,7 @@ __global__ __launch_bounds__(256) void pa_decode_kernel(PAParams p) {
       return;
     }
   }
-  decode_unit<E, D, NT, KV8, NX>(p, b);
+  decode_unit<E, D, NT, KV8, NX, LINES>(p, b);
 }
 
 // Stream-K over the prefill-class work: a flat space of (sequence, kv head, tile, chunk),
@@ -2489,7 +2471,7 @@ __global__ __launch_bounds__(256, 2) void pa_mixed_kernel(PAParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[prefill_lds_bytes<D, KV8>()];
   const int b = blockIdx.x;
   if (b < p.ND)
-    decode_unit<E, D, 1, KV8, 1>(p, b);
+    decode_unit<E, D, 1, KV8, 1, false>(p, b);
   else
     prefill_unit<E, D, KV8, false>(p, b - p.ND, lds);
 }
@@ -2570,13 +2552,13 @@ static int decode_units(PAParams& p, int resident, int per_cu, bool kv8) {
   return wgs;
 }
 
-template <class E, int D, int NT, bool KV8, int NX = 1>
+template <class E, int D, int NT, bool KV8, int NX = 1, bool LINES = false>
 static int launch_decode_nt(PAParams& p, hipStream_t s) {
   int per_cu = 1;
-  const int resident = resident_blocks((const void*)&pa_decode_kernel<E, D, NT, KV8, NX>, 256, &per_cu);
+  const int resident = resident_blocks((const void*)&pa_decode_kernel<E, D, NT, KV8, NX, LINES>, 256, &per_cu);
   const int wgs = decode_units(p, resident, per_cu, KV8);
   p.ND = p.NUP > 0 ? wgs : 0;  // NUP > 0: the workgroups behind the decode units plan the prefill launch
-  hipLaunchKernelGGL((pa_decode_kernel<E, D, NT, KV8, NX>), dim3(wgs + p.NUP), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((pa_decode_kernel<E, D, NT, KV8, NX, LINES>), dim3(wgs + p.NUP), dim3(256), 0, s, p);
   return (int)hipGetLastError();
 }
 
@@ -2584,7 +2566,11 @@ static int launch_decode_nt(PAParams& p, hipStream_t s) {
 template <class E, int D, bool KV8>
 static int launch_decode(PAParams& p, int NT, hipStream_t s) {
   switch (NT) {
-    case 1: return launch_decode_nt<E, D, 1, KV8>(p, s);
+    case 1:
+      if constexpr (line_dim(D))
+        if (p.NUP == 0 && line_launch(D, p.RS, p.k_ss * (KV8 ? 1 : 2)))
+          return launch_decode_nt<E, D, 1, KV8, 1, true>(p, s);
+      return launch_decode_nt<E, D, 1, KV8>(p, s);
     case 2: return launch_decode_nt<E, D, 2, KV8>(p, s);
     case 3: return launch_decode_nt<E, D, 3, KV8>(p, s);
     case 4: return launch_decode_nt<E, D, 4, KV8>(p, s);
@@ -2638,10 +2624,8 @@ template <class E, int D, bool KV8>
 static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipStream_t s, LaunchLog& log) {
   int err = 0;
   if (plan.short_decode) {
-    const int64_t rows = (int64_t)p.B * p.Hkv * D;
-    if (can_read_lines<D, KV8>() && (KV8 ? rows * p.W * p.BS >= kShortLines8 : rows >= kShortLines))
-      hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, can_read_lines<D, KV8>()>), dim3(p.Hkv, p.B), dim3(256), 0, s,
-                         p);
+    if (line_short(D, KV8, (int64_t)p.B * p.Hkv * D, (int64_t)p.W * p.BS))
+      hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, can_read_lines(D, KV8)>), dim3(p.Hkv, p.B), dim3(256), 0, s, p);
     else
       hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, false>), dim3(p.Hkv, p.B), dim3(256), 0, s, p);
     if ((err = (int)hipGetLastError())) return err;

@@ -1,7 +1,7 @@
 """Decode through whole-line K reads (up to 8 query rows per kv head) and past them: the short
 decode of batches large enough to take them, with stale slots that hold NaN, at row counts on
 both sides of 8, over 16-bit and E4M3 caches; and the stream-K decode on both sides of the unit
-length up to which 16-bit caches take them."""
+lengths where 16-bit and E4M3 caches take them, at row distances and query rows on both sides of theirs."""
 
 from __future__ import annotations
 
@@ -56,3 +56,47 @@ def test_stream_k_decode(hip_device, heads, q, ctx):
     out = pc.attend(b)
     assert "reduce" in last_launch_kernels()
     assert pc.max_err_vs_oracle(b, out, [0, 1, B // 2, B - 1]) <= pc.TOL_16BIT
+
+
+@pytest.mark.parametrize(("e4m3", "chunks"), [(False, 4), (False, 31), (False, 33), (True, 7), (True, 9)])
+@pytest.mark.parametrize(("heads", "q", "head_dim"), [((32, 8), [1], 128), ((32, 8), [1, 2, 3], 128), ((24, 12), [4], 128),
+                                                      ((16, 16), [1], 128), ((8, 2), [1], 128), ((32, 8), [1], 64)])  # fmt: skip
+def test_stream_k_lines(hip_device, heads, q, head_dim, e4m3, chunks):
+    """Sequences whose stale slots hold NaN, the mean unit about `chunks` chunks long; queries of 1 to 3 tokens
+    make batches whose most query rows are past 8 while some sequences' are not."""
+    H, Hkv = heads
+    hgw = 8 if Hkv % 8 == 0 else 4 if Hkv % 4 == 0 else 2
+    units = (2048 if e4m3 or head_dim == 64 else 1024) // hgw  # waves over heads a unit, on 256 CUs
+    if e4m3 and head_dim == 64:
+        units *= 2
+    rng = random.Random(chunks)
+    B = 20
+    mean = chunks * units * 32 // (B * (Hkv // hgw))
+    lens = [max(1, mean + rng.randint(-40, 40)) for _ in range(B)]
+    if max(lens) + 4 <= 1024:
+        lens[0] = 1100  # past the short decode
+    w = workloads.custom("lines", [q[i % len(q)] for i in range(B)], lens, H, Hkv, head_dim, 16, seed=3)
+    b = workloads.materialize(w, torch.bfloat16, hip_device, seed=3)
+    for t, n in zip(w.tables, w.seq_lens):
+        if n % 16:
+            b.k_cache[t[n // 16], n % 16 :] = float("nan")
+            b.v_cache[t[n // 16], n % 16 :] = float("nan")
+    kf, vf = b.k_cache, b.v_cache
+    if e4m3:
+        k, v = ((x.float() / f).clamp(-448, 448).to(fp8.FP8) for x, f in ((b.k_cache, 1.0), (b.v_cache, 0.5)))
+        HipAttention.write_kv(k, v, b.k_new, b.v_new, b.meta.slot_mapping, k_scale=1.0, v_scale=0.5)
+        out = HipAttention.forward(b.q, k, v, b.meta, w.scale, k_scale=1.0, v_scale=0.5)
+        kf, vf = k.float(), v.float() * 0.5
+    else:
+        out = pc.attend(b)
+    assert "reduce" in last_launch_kernels()
+    G, t0 = H // Hkv, 0
+    for i, (n, s) in enumerate(zip(w.query_lens, w.seq_lens)):
+        if i in (0, 7, B - 1):
+            rows = b.meta.block_tables[i, : -(-s // 16)]
+            ks, vs = (x[rows].flatten(0, 1)[:s].float().repeat_interleave(G, 1) for x in (kf, vf))
+            x = torch.einsum("qhd,khd->hqk", b.q[t0 : t0 + n].float().cpu(), ks.cpu()) * w.scale
+            hidden = torch.arange(s)[None, :] > s - n + torch.arange(n)[:, None]
+            ref = torch.einsum("hqk,khd->qhd", torch.softmax(x.masked_fill(hidden, float("-inf")), -1), vs.cpu())
+            assert (out[t0 : t0 + n].float().cpu() - ref).abs().max().item() <= pc.TOL_16BIT
+        t0 += n
