@@ -113,7 +113,7 @@ def measure(idx: int, steps: int, warmup: int, prof_iters: int, seed: int = 0, f
     from the same N(0, 1) values), K/V bytes counted at one byte per element."""
     import torch
 
-    from kvserve_amd import HipAttention, _lib, last_launch_kernels, workloads
+    from kvserve_amd import HipAttention, _lib, last_launches, workloads
 
     w = workloads.baseline_config(idx, seed=seed)
     b = workloads.materialize(w, torch.bfloat16, "cuda:0", seed=seed)
@@ -182,7 +182,7 @@ def measure(idx: int, steps: int, warmup: int, prof_iters: int, seed: int = 0, f
         flush.amax()
         lib.kvh_profile_arm(ev.array, 5)
         HipAttention.forward(b.q, b.k_cache, b.v_cache, b.meta, w.scale, **kw)
-        kinds = last_launch_kernels()
+        kinds = last_launches()
         for k, kind in enumerate(kinds[:4]):
             per_kernel.setdefault(kind, []).append(ev.elapsed_ms(k, k + 1))
     ev.close()
@@ -246,7 +246,7 @@ def measure_sweep(iters: int = 50, warmup: int = 5) -> list[dict]:
     formula and as a fraction of 8 TB/s. One JSON line per point."""
     import torch
 
-    from kvserve_amd import HipAttention, _lib, last_launch_kernels, workloads
+    from kvserve_amd import HipAttention, _lib, last_launches, workloads
 
     H, Hkv, D, BS = 32, 8, 64, 16
     flush = torch.zeros(FLUSH_BYTES // 4, dtype=torch.int32, device="cuda:0")
@@ -277,7 +277,7 @@ def measure_sweep(iters: int = 50, warmup: int = 5) -> list[dict]:
                 end.record()
                 end.synchronize()
                 times.append(start.elapsed_time(end))
-                kinds = last_launch_kernels()
+                kinds = last_launches()
                 kern.append(ev.elapsed_ms(0, len(kinds[:4])))
             ms = statistics.median(times)
             kms = statistics.median(kern)

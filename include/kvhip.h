@@ -337,7 +337,8 @@ KVH_API int kvh_gemv_silu_mul(const void* x, int64_t x_row_stride, const void* w
  * array of n <= 8 hipEvent_t handles (created by the caller with timing enabled), the NEXT
  * kvh_paged_attention call on this host thread records events[0] on its stream before its
  * first kernel and events[k] right after its k-th kernel (k = 1 .. n-1), then disarms
- * itself. The call still launches all of its work. Pass events = NULL to disarm.
+ * itself. The call launches the same kernels as when it is not timed. Pass events = NULL to
+ * disarm.
  */
 KVH_API int kvh_profile_arm(void* const* events, int32_t num_events);
 
@@ -350,6 +351,7 @@ enum kvh_kernel_kind {
   KVH_KERNEL_F32 = 4,      /* exact fp32 path */
   KVH_KERNEL_SHARE = 5,    /* shared-prefix plan of the cascade decode (long tables, decode-only batches) */
   KVH_KERNEL_VALU16 = 6,   /* 16-bit shapes the MFMA kernels do not tile (vector-ALU kernel) */
+  KVH_KERNEL_MIXED = 7,    /* decode-class work and prefill-class tiles in one launch */
 };
 KVH_API int kvh_last_launch_kernels(int32_t* kinds, int32_t cap);
 

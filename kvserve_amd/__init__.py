@@ -19,6 +19,7 @@ from kvserve_amd.attention import (
     hip_available,
     hip_eligible,
     last_launch_kernels,
+    last_launches,
 )
 
 __all__ = [
@@ -29,4 +30,5 @@ __all__ = [
     "hip_available",
     "hip_eligible",
     "last_launch_kernels",
+    "last_launches",
 ]

@@ -386,11 +386,18 @@ class HipAttention:
         return out
 
 
-def last_launch_kernels() -> list[str]:
-    """Kernel kinds launched by the last forward() on this thread, in order."""
+def last_launches() -> list[str]:
+    """The kernels launched by the last forward() on this thread, in order, one name a launch (what the
+    k-th event of kvh_profile_arm follows). "mixed": decode and prefill work in one launch."""
     buf = (ctypes.c_int32 * 8)()
     n = _lib.load().kvh_last_launch_kernels(buf, 8)
     return [_lib.KERNEL_KINDS.get(buf[i], "?") for i in range(min(n, 8))]
+
+
+def last_launch_kernels() -> list[str]:
+    """Kinds of kernel work launched by the last forward() on this thread, in order: last_launches()
+    with a "mixed" launch as its two parts."""
+    return [part for k in last_launches() for part in (("decode", "prefill") if k == "mixed" else (k,))]
 
 
 def hip_available() -> bool:

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "kvhip.h"  // kvh_kernel_kind
+
 namespace kvh {
 
 // Upper bound on the waves one decode launch uses (256 CUs x 8 waves per SIMD x 4 SIMDs

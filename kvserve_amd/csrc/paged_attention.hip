@@ -2587,8 +2587,7 @@ constexpr int64_t kFusedUnitChunks = 4;
 // two kinds of workgroup on one CU take longer together than one after the other (512 decodes
 // of 255-4095 keys beside four 384-token chunks 851 us in one launch, 816 apart; 100 decodes of
 // 255-2000 keys beside the same chunks 216 and 188; 512 decodes beside one 17-token chunk 721
-// and 741). Apart as well when the call's kernels are being timed, or when a decode row needs more
-// than one 16-row tile (GQA groups above 16).
+// and 741). Apart as well when a decode row needs more than one 16-row tile (GQA groups above 16).
 template <class E, int D, bool KV8>
 static int launch_mixed(PAParams& p, int NT, int32_t max_q, hipStream_t s, LaunchLog& log) {
   p.PR = kWavesPerWG * 16 * prefill_nt<KV8>();
@@ -2602,21 +2601,20 @@ static int launch_mixed(PAParams& p, int NT, int32_t max_q, hipStream_t s, Launc
   int err, per_cu = 1;
   const int resident = resident_blocks((const void*)&pa_mixed_kernel<E, D, KV8>, 256, &per_cu);
   const int wgs = decode_units(p, resident, per_cu, KV8);
-  if (log.events || NT > 1 || dec_chunks > kFusedUnitChunks * p.NU) {
+  if (NT > 1 || dec_chunks > kFusedUnitChunks * p.NU) {
     p.NUP = std::max(8, std::min(resident_blocks((const void*)&pa_prefill_kernel<E, D, KV8>), cap) / 8 * 8);
     if ((err = launch_decode<E, D, KV8>(p, NT, s))) return err;
-    log.after_launch(1, s);
+    log.after_launch(KVH_KERNEL_DECODE, s);
     hipLaunchKernelGGL((pa_prefill_kernel<E, D, KV8>), dim3(p.NUP), dim3(256), 0, s, p);
     if ((err = (int)hipGetLastError())) return err;
-    log.after_launch(2, s);
+    log.after_launch(KVH_KERNEL_PREFILL, s);
     return 0;
   }
   p.NUP = std::max(8, std::min(resident, cap) / 8 * 8);
   p.ND = (wgs + 7) / 8 * 8;  // prefill workgroup b keeps XCD b % 8
   hipLaunchKernelGGL((pa_mixed_kernel<E, D, KV8>), dim3(p.ND + p.NUP), dim3(256), 0, s, p);
   if ((err = (int)hipGetLastError())) return err;
-  log.after_launch(1, s);
-  log.after_launch(2, s);
+  log.after_launch(KVH_KERNEL_MIXED, s);
   return 0;
 }
 
@@ -2629,14 +2627,14 @@ static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipSt
     else
       hipLaunchKernelGGL((pa_decode_short_kernel<E, D, KV8, false>), dim3(p.Hkv, p.B), dim3(256), 0, s, p);
     if ((err = (int)hipGetLastError())) return err;
-    log.after_launch(1, s);
+    log.after_launch(KVH_KERNEL_DECODE, s);
     return 0;
   }
   p.CASC = plan.cascade ? 1 : 0;
   if (plan.cascade) {
     hipLaunchKernelGGL(pa_share_kernel, dim3(1), dim3(kPlanThreads), 0, s, p);
     if ((err = (int)hipGetLastError())) return err;
-    log.after_launch(5, s);
+    log.after_launch(KVH_KERNEL_SHARE, s);
   }
   if (plan.launch_prefill) {
     if ((err = launch_mixed<E, D, KV8>(p, plan.NT, max_q, s, log))) return err;
@@ -2645,7 +2643,7 @@ static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipSt
     err = plan.cascade && p.XR == 16 * NX ? launch_decode_nt<E, D, 1, KV8, NX>(p, s)
                                           : launch_decode<E, D, KV8>(p, plan.NT, s);
     if (err) return err;
-    log.after_launch(1, s);
+    log.after_launch(KVH_KERNEL_DECODE, s);
   }
   const int mr = plan.launch_prefill ? merge_rows_decode<D, true>() : merge_rows_decode<D, false>();
   const int cd = (p.HGW * p.RS + mr - 1) / mr;
@@ -2660,7 +2658,7 @@ static int launch_mfma_typed(PAParams& p, const Plan& plan, int32_t max_q, hipSt
   else
     hipLaunchKernelGGL((pa_merge_kernel<E, D, false, false>), mg, dim3(256), 0, s, p);
   if ((err = (int)hipGetLastError())) return err;
-  log.after_launch(3, s);
+  log.after_launch(KVH_KERNEL_REDUCE, s);
   return 0;
 }
 

@@ -147,7 +147,7 @@ int launch_paged_attention_valu(const PAParams& p, int32_t D, int32_t dtype, int
     err = launch_valu<Half16<kvh::F16>>(p, D, max_q, s);
   else
     err = launch_valu<Half16<BF16>>(p, D, max_q, s);
-  if (!err) log.after_launch(dtype == 0 ? 4 : 6, s);
+  if (!err) log.after_launch(dtype == 0 ? KVH_KERNEL_F32 : KVH_KERNEL_VALU16, s);
   return err;
 }
 
