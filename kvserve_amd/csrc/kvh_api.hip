@@ -71,8 +71,9 @@ Plan make_plan(int64_t T, int32_t B, int32_t H, int32_t Hkv, int32_t D, int32_t 
     const size_t prows = pl.launch_prefill ? (size_t)2 * kMaxPrefillUnits * kPrefillRows : 0;
     pl.ws_pacc_bytes = align_up(prows * D * sizeof(float));
     pl.ws_pml_bytes = align_up(prows * 2 * sizeof(float));
-    // where each prefill unit starts, behind a header and two per-sequence arrays that no kernel
-    // uses any more: callers size their workspaces by this sum, which stays
+    // where each prefill unit starts; the sum also counts a header and two per-sequence arrays (12 bytes a
+    // sequence) that no kernel reads or writes: the size of every shape is fixed by the host tests, so that
+    // a size a caller computed or saved earlier stays right
     pl.ws_plan_bytes = pl.launch_prefill ? align_up(4 * sizeof(int64_t)) + align_up((size_t)B * sizeof(int32_t)) +
                                                align_up(((size_t)B + 1) * sizeof(int64_t)) +
                                                align_up((size_t)kMaxPrefillUnits * kPreStartBytes)

@@ -44,6 +44,7 @@
 namespace kvh {
 
 constexpr int kChunk = 32;  // tokens per wave iteration
+static_assert(kPlanChunk == kChunk, "the prefill plan counts the tiles' chunks");
 constexpr int kWavesPerWG = 4;
 // 16-row tiles per prefill wave: 3 over 16-bit caches (48 rows, 238 VGPRs at D = 128, 2 workgroups per
 // CU), 2 over E4M3 caches (whose conversion registers leave no room for a third)
@@ -2491,7 +2492,7 @@ static int resident_blocks(const void* kernel, int block_threads = 256, int* per
     const void* kernel;
     int blocks, per_cu;
   };
-  static thread_local Entry cache[16];
+  static thread_local Entry cache[64];  // every kernel of a dtype, head size and cache type, on several devices
   static thread_local int cache_n = 0;
   for (int i = 0; i < cache_n; ++i)
     if (cache[i].dev == dev && cache[i].kernel == kernel) {
@@ -2503,7 +2504,7 @@ static int resident_blocks(const void* kernel, int block_threads = 256, int* per
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block_threads, 0) != hipSuccess || per_cu <= 0)
     per_cu = 1;
   const int blocks = cus * per_cu;
-  if (cache_n < 16) cache[cache_n++] = Entry{dev, kernel, blocks, per_cu};
+  if (cache_n < 64) cache[cache_n++] = Entry{dev, kernel, blocks, per_cu};
   if (per_cu_out) *per_cu_out = per_cu;
   return blocks;
 }
