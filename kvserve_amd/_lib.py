@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 import torch  # noqa: F401  (see module docstring: must precede the CDLL load)
@@ -171,22 +172,37 @@ def load() -> ctypes.CDLL:
                 f"kvserve_amd/_kvhfast is not built ({e}): build it with `python -m kvserve_amd.build`."
             ) from e
         global _calls
-        import torch  # the libraries _kvhtorch links to
-
-        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw_stream is not None:
-            try:
-                from kvserve_amd import _kvhtorch
-            except ImportError as e:
-                raise RuntimeError(
-                    f"kvserve_amd/_kvhtorch is not built ({e}): build it with `python -m kvserve_amd.build`."
-                ) from e
-            _kvhtorch.bind(lib._handle, raw_stream)
-            _calls = _kvhtorch
+        _calls = _tensor_calls(lib)
         _kvhfast.bind(lib._handle)
         _fast = _kvhfast
         _lib = lib
     return _lib
+
+
+def _tensor_calls(lib: ctypes.CDLL):
+    """_kvhtorch bound to `lib`, or None: it only saves host time (HipAttention's methods make the same calls
+    through _kvhfast), and it holds the tensor layout of the PyTorch it was compiled against, so it is used with
+    that one alone."""
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw_stream is None:  # a build without a GPU backend
+        return None
+    try:
+        from kvserve_amd import _kvhtorch
+    except ImportError as e:
+        why = f"is not built ({e})"
+    else:
+        built = getattr(_kvhtorch, "torch_version", "unknown")
+        if built == str(torch.__version__):
+            _kvhtorch.bind(lib._handle, raw_stream)
+            return _kvhtorch
+        why = f"was built for PyTorch {built}, not {torch.__version__}"
+    warnings.warn(
+        f"kvserve_amd/_kvhtorch {why}: calls take about 10 us more host time. Build it with "
+        "`python -m kvserve_amd.build`.",
+        RuntimeWarning,
+        stacklevel=4,
+    )
+    return None
 
 
 def fast():
@@ -197,8 +213,8 @@ def fast():
 
 
 def calls():
-    """The per-step calls on tensors (_kvhtorch), bound to the loaded library; None when this PyTorch
-    does not hand out stream handles (a build without a GPU backend)."""
+    """The per-step calls on tensors (_kvhtorch), bound to the loaded library; None where they cannot be used
+    (_tensor_calls)."""
     if _lib is None:
         load()
     return _calls

@@ -122,6 +122,7 @@ def build_torch_calls(verbose: bool = False) -> Path:
     tmp = out.with_suffix(".so.tmp")
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+           f'-DKVH_TORCH_VERSION="{torch.__version__}"',
            f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", *[f"-isystem{d}" for d in include_paths()],
            str(CSRC / "pytorch_calls.cpp"), *[f"-L{d}" for d in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10",
            "-ldl", "-o", str(tmp)]  # fmt: skip
@@ -182,7 +183,12 @@ def build(
     os.replace(tmp, lib)  # atomic: a process that already mapped the old file keeps it
     if out is None:
         build_fastcall(verbose)
-        build_torch_calls(verbose)
+        try:
+            build_torch_calls(verbose)
+        except RuntimeError as e:  # only host time is lost without it: the Python methods make the same calls
+            print(f"_kvhtorch is not built: {e}", file=sys.stderr)
+            for old in PKG.glob("_kvhtorch*.so"):  # never an older build of it beside the new library
+                old.unlink()
     return lib
 
 

@@ -11,6 +11,8 @@
 // Python number) the functions return None before any work, and the Python method does what it
 // always did, its error included. They return the output tensor (True for write_kv), or the nonzero
 // status of the C ABI. Nothing is kept between calls but the entry points that bind() resolves.
+// Without this module the Python methods do everything: it is left out where it was built for another
+// PyTorch (torch_version).
 #include <Python.h>
 #include <dlfcn.h>
 
@@ -309,4 +311,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_kvhtorch", "HipAttention's per-st
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__kvhtorch(void) { return PyModule_Create(&module); }
+// torch_version: the PyTorch this was compiled against, which alone it may be used with
+PyMODINIT_FUNC PyInit__kvhtorch(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", KVH_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}
