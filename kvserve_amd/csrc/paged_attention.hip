@@ -1160,7 +1160,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
                         rounds ? kRound1Share : 1, rounds ? kRound2Share : 1);
   const int64_t a = split.begin(unit), b = split.begin(unit + 1);
   if (a >= b) return;
-  const bool lines = LINES && L == 0 && line_units(KV8, C, NUa);
+  const bool lines = LINES && line_units(KV8, C, NUa);
 
   int64_t pos = a;
   if constexpr (NT == 1) {
