@@ -85,6 +85,7 @@ struct PAParams {
   float* ws_xacc;        // [xslots, HGW, XR, D] partials of the prefix segments
   float* ws_xml;         // [xslots, HGW, XR, 2]
   int32_t* ws_xjob;      // [B * Hkv / HGW, kJobInts] merge jobs per (sequence, head group)
+  int32_t LINES;         // mixed batch in one launch: K's token rows lie where whole-line reads pay
 };
 
 // Launch plan: a pure function of static shapes (graph-capture safe).

@@ -13,19 +13,19 @@ namespace kvh {
 constexpr bool can_read_lines(int D, bool kv8) { return !kv8 || D == 128; }
 constexpr int kLineRows = 8;  // query rows they serve
 
-// The stream-K decode of a decode-only batch. It takes them for all units of a launch or for none: with
-// both kinds on one CU the units ran up to 15% longer than with either kind alone (50 sequences of 2600 keys, 8
-// kv heads, 8 query rows, 32.0 chunks a unit with a limit of 32 on each unit's own length: 98.2 / 112.0; one
-// sequence in ten with 12 query rows among those with 4, 24 chunks a unit: 75.1 / 81.5). So the launcher looks at the batch's
-// most query rows and the bytes between K's token rows, the kernel at the mean unit. (A cascade's prefix segments
-// keep half lines, which other groups' reads hit in the caches, and its members' own keys whole ones: 4
-// sequences over 13000 shared keys 47.6 / 46.0.)
+// The stream-K decode takes them for all units of a launch or for none: with both kinds on one CU the units
+// ran up to 15% longer than with either kind alone (50 sequences of 2600 keys, 8 kv heads, 8 query rows, 32.0
+// chunks a unit with a limit of 32 on each unit's own length: 98.2 / 112.0; one sequence in ten with 12 query
+// rows among those with 4, 24 chunks a unit: 75.1 / 81.5). So the launcher looks at the bytes between K's token
+// rows and at a decode-only batch's most query rows, the kernel at the mean unit and, beside prompt chunks, at
+// its sequences' rows. (A cascade's prefix segments keep half lines, which other groups' reads hit in the
+// caches, and its members' own keys whole ones: 4 sequences over 13000 shared keys 47.6 / 46.0.)
 constexpr bool line_dim(int D) { return D == 128; }  // D = 64, one line a row: 1-4% lost in short units
 
 // Token rows 1 to under 4 KB apart: 4, 8 or 12 kv heads of a 16-bit cache, 8, 12 or 16 of an E4M3 one. 16-bit,
 // 16 chunks a unit: 8 kv heads 54.4 / 53.4, 12 56.0 / 54.2, 4 55.0 / 54.4; 16 kv heads 53.0 / 53.8, 32 2%
-// slower (rows 4 KB apart meet in one channel), 1 and 2 1-2% slower. E4M3: 8 59.2 / 58.5, 12 5% faster; 2, 4
-// and 32 1-3% slower.
+// slower (perhaps because rows 4 KB apart meet in one channel), 1 and 2 1-2% slower. E4M3: 8 59.2 / 58.5,
+// 12 5% faster; 2, 4 and 32 1-3% slower. rows: the most query rows of a sequence (0: the kernel looks).
 KVH_LINE_FN bool line_launch(int D, int rows, int64_t row_bytes) {
   return line_dim(D) && rows <= kLineRows && row_bytes >= 1024 && row_bytes < 4096;
 }

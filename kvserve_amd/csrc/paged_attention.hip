@@ -1107,7 +1107,7 @@ __device__ __forceinline__ void write_job_x(int32_t* job, int pieces, int64_t sl
 // group (XR = 16 NX rows; 1 outside the cascade).
 // LINES: whole-line K reads where the launch's mean unit asks for them (line_units).
 template <class E, int D, int NT, bool KV8, int NX, bool LINES>
-__device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
+__device__ __forceinline__ void decode_unit(const PAParams& p, int block, bool may_read_lines = true) {
   static_assert(!LINES || (NT == 1 && NX == 1));
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1145,11 +1145,13 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
 
   // Chunks per segment over all sequences (every wave computes the sum itself).
   int Cs = 0, Ns = 0;
+  uint64_t wide = 0;  // sequences past the rows that whole-line reads serve
   for (int blk0 = 0; blk0 < p.B; blk0 += 64) {
     SeqWindow sw;
     scan_window(sw, p, blk0, Cs, Ns, L);
     Cs += sw.total;
     Ns += sw.ntotal;
+    if constexpr (LINES) wide |= __builtin_amdgcn_ballot_w64(sw.c > 0 && sw.ql * p.G > kLineRows);
   }
   const int64_t C = P + (int64_t)Cs * NHG;
   const int64_t NUa = active_units(C, p.NU);
@@ -1160,7 +1162,7 @@ __device__ __forceinline__ void decode_unit(const PAParams& p, int block) {
                         rounds ? kRound1Share : 1, rounds ? kRound2Share : 1);
   const int64_t a = split.begin(unit), b = split.begin(unit + 1);
   if (a >= b) return;
-  const bool lines = LINES && line_units(KV8, C, NUa);
+  const bool lines = LINES && may_read_lines && wide == 0 && line_units(KV8, C, NUa);
 
   int64_t pos = a;
   if constexpr (NT == 1) {
@@ -2472,7 +2474,7 @@ __global__ __launch_bounds__(256, 2) void pa_mixed_kernel(PAParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[prefill_lds_bytes<D, KV8>()];
   const int b = blockIdx.x;
   if (b < p.ND)
-    decode_unit<E, D, 1, KV8, 1, false>(p, b);
+    decode_unit<E, D, 1, KV8, 1, line_dim(D) && !KV8>(p, b, p.LINES);  // (E4M3: its units are too short for lines)
   else
     prefill_unit<E, D, KV8, false>(p, b - p.ND, lds);
 }
@@ -2569,7 +2571,7 @@ static int launch_decode(PAParams& p, int NT, hipStream_t s) {
   switch (NT) {
     case 1:
       if constexpr (line_dim(D))
-        if (p.NUP == 0 && line_launch(D, p.RS, p.k_ss * (KV8 ? 1 : 2)))
+        if (line_launch(D, p.NUP > 0 ? 0 : p.RS, p.k_ss * (KV8 ? 1 : 2)))
           return launch_decode_nt<E, D, 1, KV8, 1, true>(p, s);
       return launch_decode_nt<E, D, 1, KV8>(p, s);
     case 2: return launch_decode_nt<E, D, 2, KV8>(p, s);
@@ -2612,6 +2614,7 @@ static int launch_mixed(PAParams& p, int NT, int32_t max_q, hipStream_t s, Launc
     return 0;
   }
   p.NUP = std::max(8, std::min(resident, cap) / 8 * 8);
+  p.LINES = line_launch(D, 0, p.k_ss * (KV8 ? 1 : 2));
   p.ND = (wgs + 7) / 8 * 8;  // prefill workgroup b keeps XCD b % 8
   hipLaunchKernelGGL((pa_mixed_kernel<E, D, KV8>), dim3(p.ND + p.NUP), dim3(256), 0, s, p);
   if ((err = (int)hipGetLastError())) return err;
