@@ -10,7 +10,7 @@ import random
 import pytest
 import torch
 
-from kvserve_amd import HipAttention, last_launch_kernels, workloads
+from kvserve_amd import HipAttention, last_launch_kernels, last_launches, workloads
 from oracle import fp8, torch_reference
 from tests import paged_check as pc
 
@@ -81,18 +81,26 @@ def test_stream_k_lines(hip_device, heads, q, head_dim, e4m3, chunks):
         if n % 16:
             b.k_cache[t[n // 16], n % 16 :] = float("nan")
             b.v_cache[t[n // 16], n % 16 :] = float("nan")
-    kf, vf = b.k_cache, b.v_cache
-    if e4m3:
-        k, v = ((x.float() / f).clamp(-448, 448).to(fp8.FP8) for x, f in ((b.k_cache, 1.0), (b.v_cache, 0.5)))
-        HipAttention.write_kv(k, v, b.k_new, b.v_new, b.meta.slot_mapping, k_scale=1.0, v_scale=0.5)
-        out = HipAttention.forward(b.q, k, v, b.meta, w.scale, k_scale=1.0, v_scale=0.5)
-        kf, vf = k.float(), v.float() * 0.5
-    else:
-        out = pc.attend(b)
+    out, kf, vf = _attend(b, e4m3)
     assert "reduce" in last_launch_kernels()
-    G, t0 = H // Hkv, 0
+    _check(b, out, kf, vf, (0, 7, B - 1))
+
+
+def _attend(b, e4m3):
+    """The batch's attention, over the caches or over them in E4M3, and the values that they hold."""
+    if not e4m3:
+        return pc.attend(b), b.k_cache, b.v_cache
+    k, v = ((x.float() / f).clamp(-448, 448).to(fp8.FP8) for x, f in ((b.k_cache, 1.0), (b.v_cache, 0.5)))
+    HipAttention.write_kv(k, v, b.k_new, b.v_new, b.meta.slot_mapping, k_scale=1.0, v_scale=0.5)
+    out = HipAttention.forward(b.q, k, v, b.meta, b.workload.scale, k_scale=1.0, v_scale=0.5)
+    return out, k.float(), v.float() * 0.5
+
+
+def _check(b, out, kf, vf, seqs):
+    w = b.workload
+    G, t0 = w.num_heads // w.num_kv_heads, 0
     for i, (n, s) in enumerate(zip(w.query_lens, w.seq_lens)):
-        if i in (0, 7, B - 1):
+        if i in seqs:
             rows = b.meta.block_tables[i, : -(-s // 16)]
             ks, vs = (x[rows].flatten(0, 1)[:s].float().repeat_interleave(G, 1) for x in (kf, vf))
             x = torch.einsum("qhd,khd->hqk", b.q[t0 : t0 + n].float().cpu(), ks.cpu()) * w.scale
@@ -100,3 +108,17 @@ def test_stream_k_lines(hip_device, heads, q, head_dim, e4m3, chunks):
             ref = torch.einsum("hqk,khd->qhd", torch.softmax(x.masked_fill(hidden, float("-inf")), -1), vs.cpu())
             assert (out[t0 : t0 + n].float().cpu() - ref).abs().max().item() <= pc.TOL_16BIT
         t0 += n
+
+
+@pytest.mark.parametrize("decodes", [6, 90])  # one launch with the chunk's tiles, a launch of their own
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("q", [[1], [2], [1, 2, 4], [4]])
+def test_beside_a_prompt_chunk(hip_device, q, e4m3, decodes):
+    """Decoding sequences beside a prompt chunk, all of them up to 8 query rows, some, or none."""
+    rng = random.Random(decodes)
+    n = [q[i % len(q)] for i in range(decodes)]
+    w = workloads.custom("beside", [*n, 130], [rng.randint(900, 1500) for _ in n] + [70], 32, 8, 128, 16, seed=4)
+    b = workloads.materialize(w, torch.bfloat16, hip_device, seed=4)
+    out, kf, vf = _attend(b, e4m3)
+    assert last_launches() == (["mixed", "reduce"] if decodes == 6 else ["decode", "prefill", "reduce"])
+    _check(b, out, kf, vf, (0, 1, 2, decodes - 1, decodes))
