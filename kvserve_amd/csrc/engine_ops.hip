@@ -298,7 +298,7 @@ int launch_gemv_t(const void* x, int64_t x_rs, const void* w, int64_t w_rs, void
 // gate rows c0 + i, the others the up rows inter + c0 + i; the epilogue rounds each sum to the
 // storage type and applies silu_mul's arithmetic (the bits of the plain kernel followed by
 // kvh_silu_mul). n is then the intermediate size.
-template <class E, SkinnyForm F, int MT, bool GLU>
+template <class E, SkinnyForm F, int MT, bool GLU, bool ONE = false>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_rs,
                                                                         const uint16_t* __restrict__ w, int64_t w_rs,
                                                                         uint16_t* __restrict__ y, int64_t y_rs, int m,
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(const ui
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  skinny_slice<E, F, MT>(wr, x, x_rs, m, ks, slice, len, lds, acc);
+  skinny_slice<E, F, MT, ONE>(wr, x, x_rs, m, ks, slice, len, lds, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
@@ -355,12 +355,21 @@ int launch_skinny_t(const void* x, int64_t x_rs, const void* w, int64_t w_rs, vo
   const int tiles = (int)(rows / skinny_rows(skinny_form(rows, k, m)));
   const dim3 grid((unsigned)((tiles + per - 1) / per)), block(64 * kSkinnyWaves);
   const int vec = (((uintptr_t)y | (uintptr_t)(2 * y_rs)) & 7) == 0;  // 8-byte stores
-#define KVH_LAUNCH_SKINNY(F, MT)                                                                                    \
-  hipLaunchKernelGGL((skinny_gemm_kernel<E, F, MT, GLU>), grid, block, (skinny_lds_bytes<F, MT>(ks)), s,             \
+#define KVH_LAUNCH_SKINNY(F, MT, ...)                                                                               \
+  hipLaunchKernelGGL((skinny_gemm_kernel<E, F, MT, GLU, ##__VA_ARGS__>), grid, block, (skinny_lds_bytes<F, MT>(ks)), s,             \
                      (const uint16_t*)x, x_rs, (const uint16_t*)w, w_rs, (uint16_t*)y, y_rs, m, k, n, ks, vec)
   switch (skinny_form(rows, k, m)) {
     case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
     case kSkinnyFull:
+      if (k == 1024) {  // one batch a slice
+        switch ((m + 15) / 16) {
+          case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1, true); break;
+          case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2, true); break;
+          case 3: KVH_LAUNCH_SKINNY(kSkinnyFull, 3, true); break;
+          default: KVH_LAUNCH_SKINNY(kSkinnyFull, 4, true); break;
+        }
+        break;
+      }
       switch ((m + 15) / 16) {
         case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1); break;
         case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2); break;

@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256) void gemv_rope_cache_kernel(GemvRopeArgs a) {
 // engine_ops.hip): `ks` waves (k-slices) own NP = 8 or 4 pairs, one A tile of rows h D + d0 + i for
 // i < NP, h D + d0 + D / 2 + i - NP for i >= NP, and MT B tiles of x; the partial tiles meet in LDS,
 // are summed in slice order and go through rope_pair_out.
-template <int DT, SkinnyForm F, int MT, bool KV8>
+template <int DT, SkinnyForm F, int MT, bool KV8, bool ONE = false>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(GemvRopeArgs a, int m, int slices) {
   using E = std::conditional_t<DT == 2, BF16, F16>;
   constexpr int THREADS = 64 * kSkinnyWaves, TR = skinny_rows(F), NP = TR / 2;
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_rope_cache_kernel(Ge
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  skinny_slice<E, F, MT>(wr, a.x, a.x_rs, m, ks, slice, len, lds, acc);
+  skinny_slice<E, F, MT, ONE>(wr, a.x, a.x_rs, m, ks, slice, len, lds, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
@@ -361,11 +361,20 @@ static int launch_gemv_rope_dt(const GemvRopeArgs& a, int m, hipStream_t s) {
     const int ks = skinny_slices(rows, a.k, m), per = kSkinnyWaves / ks;
     const int tiles = (int)(rows / skinny_rows(skinny_form(rows, a.k, m)));
     const dim3 g2((unsigned)((tiles + per - 1) / per)), b2(64 * kSkinnyWaves);
-#define KVH_LAUNCH_SKINNY(F, MT) \
-  hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, F, MT, KV8>), g2, b2, (skinny_lds_bytes<F, MT>(ks)), s, a, m, ks)
+#define KVH_LAUNCH_SKINNY(F, MT, ...) \
+  hipLaunchKernelGGL((skinny_rope_cache_kernel<DT, F, MT, KV8, ##__VA_ARGS__>), g2, b2, (skinny_lds_bytes<F, MT>(ks)), s, a, m, ks)
     switch (skinny_form(rows, a.k, m)) {
       case kSkinnyHalf: KVH_LAUNCH_SKINNY(kSkinnyHalf, 1); break;
       case kSkinnyFull:
+        if (a.k == 1024) {  // one batch a slice
+          switch ((m + 15) / 16) {
+            case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1, true); break;
+            case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2, true); break;
+            case 3: KVH_LAUNCH_SKINNY(kSkinnyFull, 3, true); break;
+            default: KVH_LAUNCH_SKINNY(kSkinnyFull, 4, true); break;
+          }
+          break;
+        }
         switch ((m + 15) / 16) {
           case 1: KVH_LAUNCH_SKINNY(kSkinnyFull, 1); break;
           case 2: KVH_LAUNCH_SKINNY(kSkinnyFull, 2); break;

@@ -47,14 +47,17 @@ __device__ __forceinline__ int skinny_k(int lane) {
 // acc[t] += (x rows of B tile t) . (the tile's weight rows) over slice `slice` of the
 // workgroup's ks, `len` of k (whole batches, or chunks). wr: this lane's first elements of the
 // weight; x, x_rs, m: the rows of x (past m, row m - 1 is read); lds: skinny_lds_bytes.
-template <class E, SkinnyForm F, int MT>
+// ONE: a slice is one batch (full tiles at k = 1024), with no second set of registers: 38 instead of 82 at
+// 16 rows of x, so the workgroups of up to 16384 weight rows fit the chip at once ((12288, 1024) at 5 rows 8.9 us,
+// so 6.9).
+template <class E, SkinnyForm F, int MT, bool ONE>
 __device__ __forceinline__ void skinny_slice(const uint16_t* wr, const uint16_t* x, int64_t x_rs, int m, int ks,
                                              int slice, int len, char* lds, f32x4 (&acc)[MT]) {
   constexpr int U = 4, STEP = skinny_step(F), BATCH = skinny_batch(F), ROWS = skinny_rows(F) * MT;
   const int lane = threadIdx.x & 63;
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
-  u32x4 a[2][U];
+  u32x4 a[ONE ? 1 : 2][U];
   auto load_a = [&](auto S, int kk) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -77,7 +80,7 @@ __device__ __forceinline__ void skinny_slice(const uint16_t* wr, const uint16_t*
 #pragma unroll
     for (int t = 0; t < MT; ++t)
       xr[t] = x + (int64_t)min(skinny_rows(F) * t + skinny_row<F>(lane), m - 1) * x_rs + slice * len + skinny_k<F>(lane);
-    u32x4 b[2][U][MT];
+    u32x4 b[ONE ? 1 : 2][U][MT];
     auto load = [&](auto S, int kk) {
       load_a(S, kk);
 #pragma unroll
@@ -87,19 +90,23 @@ __device__ __forceinline__ void skinny_slice(const uint16_t* wr, const uint16_t*
       __builtin_amdgcn_sched_barrier(0);
     };
     load(S0{}, 0);
-    int kk = 0;
-    for (; kk + 2 * BATCH < len; kk += 2 * BATCH) {
-      load(S1{}, kk + BATCH);
+    if constexpr (ONE) {
       mfmas(S0{}, b[0]);
-      load(S0{}, kk + 2 * BATCH);
-      mfmas(S1{}, b[1]);
-    }
-    if (kk + BATCH < len) {
-      load(S1{}, kk + BATCH);
-      mfmas(S0{}, b[0]);
-      mfmas(S1{}, b[1]);
     } else {
-      mfmas(S0{}, b[0]);
+      int kk = 0;
+      for (; kk + 2 * BATCH < len; kk += 2 * BATCH) {
+        load(S1{}, kk + BATCH);
+        mfmas(S0{}, b[0]);
+        load(S0{}, kk + 2 * BATCH);
+        mfmas(S1{}, b[1]);
+      }
+      if (kk + BATCH < len) {
+        load(S1{}, kk + BATCH);
+        mfmas(S0{}, b[0]);
+        mfmas(S1{}, b[1]);
+      } else {
+        mfmas(S0{}, b[0]);
+      }
     }
   } else {
     constexpr int VPR = kSkinnyChunk / 8, THREADS = 64 * kSkinnyWaves;

@@ -15,18 +15,20 @@ enum SkinnyForm { kSkinnyFull, kSkinnyHalf, kSkinnyShared };
 //    (3072, 2048) 6.7 / 6.1, (3072, 4096) 10.3 / 9.1, (4096, 4096) 10.4 / 9.5. Shared x from 5120 rows: (5120,
 //    2048) shared 7.9 / full 9.1 / half 9.8, (6144, 4096) 13.4 / 15.7 / 14.5; (4096, 4096) has too few tiles.
 //  * m <= 32, shared x from 8192 rows: (8192, 4096) at 16 rows 15.7 / full 18.1.
-//  * Up to 8192 rows a k of 1024 leaves each slice one chunk and nothing to load ahead: (8192, 1024) at 5
-//    rows shared 6.6 / full 5.7, at 16 rows 7.1 / 6.7; past them full tiles no longer fit the chip at once.
+//  * k = 1024 leaves each slice one chunk and nothing to load ahead, while the full tiles' slices are one
+//    batch in few registers: (8192, 1024) at 5 rows shared 6.6 / full 5.8, (12288, 1024) 8.0 / 6.9, at 12 8.7 / 8.0, at
+//    24 9.3 / 10.2; (16384, 1024) at 5 9.1 / 8.4, at 16 9.7 / 10.4.
 //  * m > 32: k stays whole (its LDS), so 8192 rows give shared x 128 workgroups: (8192, 2048) at 33 rows
 //    shared 19.5 / full 15.0, (8192, 4096) at 48 34.2 / 31.8, at 56 34.8 / 36.1; (9216, 2048) at 33 19.8 / 23.1.
 inline SkinnyForm skinny_form(int64_t rows, int64_t k, int m) {
+  if (m <= 8 && rows <= 2048 && k % 2048 == 0) return kSkinnyHalf;
   bool shared;
-  if (m <= 32) {
-    if (m <= 8 && rows <= 2048 && k % 2048 == 0) return kSkinnyHalf;
-    shared = rows >= (m <= 8 ? 5120 : 8192) && (k >= 2048 || rows > 8192);
-  } else {
+  if (k < 2048)
+    shared = rows > (m <= 8 ? 16384 : m <= 16 ? 12288 : 8192);
+  else if (m <= 32)
+    shared = rows >= (m <= 8 ? 5120 : 8192);
+  else
     shared = rows > 8192 || (rows == 8192 && m > 48);
-  }
   return shared ? kSkinnyShared : kSkinnyFull;
 }
 // weight rows (and x rows of a B tile) of a tile, k per MFMA step and per batch of 4 steps, k of a
@@ -37,8 +39,8 @@ constexpr int skinny_batch(SkinnyForm f) { return 4 * skinny_step(f); }
 constexpr int kSkinnyChunk = 512;
 
 // k-slices per tile: kSkinnyWaves, a constant of the full and half kernels (known only at run time, the sum
-// of the slices was a chain of LDS latencies: (2048, 1024) at 8 rows 4.3 us, now 4.1); with x shared
-// 2, or 1 where 2 would only add a round of workgroups (256 CUs; (10240, 1024) at 16 rows 8.4 / 10.1) or above 32
+// of the slices was a chain of LDS latencies: (2048, 1024) at 8 rows 4.3 us, so 4.1); with x shared
+// 2, or 1 where 2 would only add a round of workgroups (256 CUs; (10240, 1024) at 24 rows 9.0 / 13.2) or above 32
 // rows (its LDS).
 inline int skinny_slices(int64_t rows, int64_t k, int m) {
   if (skinny_form(rows, k, m) != kSkinnyShared) return kSkinnyWaves;

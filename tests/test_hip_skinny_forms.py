@@ -39,9 +39,9 @@ def test_gemm_skinny_forms(hip_device, m, n, k):
     assert torch.equal(z, got)
 
 
-@pytest.mark.parametrize("m", [5, 8, 9, 48, 49])
+@pytest.mark.parametrize("m", [5, 8, 9, 17, 33, 48, 49])
 @pytest.mark.parametrize(("n", "k"), [(2048, 1024), (2048, 2048), (2064, 2048), (5104, 2048), (5120, 1024), (5120, 2048),
-                                      (8192, 2048), (8208, 1024), (10240, 2048)])  # fmt: skip
+                                      (8192, 2048), (8208, 1024), (10240, 2048), (12304, 1024), (16400, 1024)])  # fmt: skip
 def test_lines_between_forms(hip_device, m, n, k):
     """Both sides of the lines that rows of the weight, k and rows of x draw between the forms, fused with RoPE
     and the cache write (the same bits as the projection and the separate step) and alone."""

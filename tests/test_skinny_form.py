@@ -48,7 +48,9 @@ MEASURED = [
     ((2048, 2048), 8, HALF), ((1024, 4096), 8, HALF), ((2048, 8192), 5, HALF), ((512, 3072), 8, FULL),
     ((3072, 2048), 8, FULL), ((3072, 4096), 8, FULL), ((4096, 4096), 8, FULL), ((2048, 1024), 8, FULL),
     ((5120, 2048), 5, SHARED), ((6144, 2048), 8, SHARED), ((6144, 4096), 8, SHARED), ((6144, 1024), 8, FULL),
-    ((8192, 1024), 5, FULL), ((8192, 1024), 16, FULL), ((8192, 1024), 40, FULL), ((10240, 1024), 16, SHARED),
+    ((8192, 1024), 5, FULL), ((8192, 1024), 16, FULL), ((8192, 1024), 64, FULL), ((10240, 1024), 24, SHARED),
+    ((12288, 1024), 5, FULL), ((12288, 1024), 12, FULL), ((14336, 1024), 16, SHARED), ((16384, 1024), 5, FULL),
+    ((16384, 1024), 16, SHARED), ((28672, 1024), 8, SHARED),
     ((8192, 4096), 16, SHARED), ((8192, 2048), 33, FULL), ((8192, 4096), 48, FULL), ((8192, 4096), 64, SHARED),
     ((9216, 2048), 33, SHARED), ((16384, 2048), 64, SHARED), ((128256, 4096), 32, SHARED),
 ]  # fmt: skip
@@ -60,7 +62,7 @@ def test_measured_shapes_take_the_faster_form(lib, shape, m, form):
 
 
 def test_extra_rounds_are_not_bought(lib):
-    assert lib.slices(8192, 4096, 16) == 2 and lib.slices(10240, 1024, 16) == 1 and lib.slices(8208, 4096, 33) == 1
+    assert lib.slices(8192, 4096, 16) == 2 and lib.slices(10240, 1024, 24) == 1 and lib.slices(8208, 4096, 33) == 1
 
 
 def test_every_choice_can_run(lib):
